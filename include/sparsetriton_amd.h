@@ -543,14 +543,21 @@ int st_gather_gemm(const void* A, int64_t n_src, const int32_t* map, int64_t map
  * the same reference kernels (implicit_precomputed_gemm.py:64-177) --:
  * the workgroup reads its tile's offsets and source rows contiguously
  * instead of gathering map entries and masks row by row.  Same result as
- * st_gather_gemm with that map.  Reductions wider than 128 (16-bit and
+ * st_gather_gemm with that map (up to fp32 rounding for reductions below 32:
+ * several offsets then share a matrix instruction).  Reductions wider than 128 (16-bit and
  * ST_F32_BF16X3) or 64 (ST_F32) return ST_ERR_UNSUPPORTED.  flags:
  * ST_GATHER_REVERSE_K multiplies offset k's sources by Bt[K - 1 - k] -- the
  * input gradient of a submanifold map that is its own transpose, read over
  * the forward's plan with the weights as given (W (K, C_in, C_out) is then
  * the Bt operand), with no ST_W_REVERSE copy: the same result bit for bit.
+ * ST_GATHER_B_KN: Bt is the layer's W (K, Kd, Nd) as it is stored, not its
+ * (K, Nd, Kd) transpose, so the forward needs no ST_W_TRANSPOSE copy; taken
+ * where st_gather_b_kn_ok says 1 (narrow layers, whose kernel lays the weights
+ * out in LDS itself), ST_ERR_UNSUPPORTED elsewhere.  Host arithmetic only: it
+ * touches no device.  No reference counterpart.
  */
-enum st_gather_flags { ST_GATHER_REVERSE_K = 1 };
+enum st_gather_flags { ST_GATHER_REVERSE_K = 1, ST_GATHER_B_KN = 2 };
+int st_gather_b_kn_ok(const void* A, int64_t n_src, int64_t n_dst, int K, int Kd, int Nd, int dtype);
 int st_gather_gemm_tiled(const void* A, int64_t n_src, const int32_t* perm, const int32_t* tile_nk,
                          const int16_t* tile_klist, const int32_t* tile_map, const void* Bt, const void* bias,
                          void* out, int64_t n_dst, int K, int Kd, int Nd, int dtype, int flags, st_stream_t stream);

@@ -1591,6 +1591,7 @@ static bool gather_lines() {
 
 }  // namespace st
 
+#include "gemm_narrow.h"
 #include "gemm_wide.h"
 
 namespace st {
@@ -1680,6 +1681,17 @@ static int launch_gather_e(const T* A, int64_t n_src, const Src& src, const uint
 
 // The general store epilogue (affine map, residual, ReLU) runs on the tiled
 // kernels only; everything else stores acc + bias.
+// Kernels that hold the whole weight tensor in LDS take the narrow layers of a
+// tile plan (gemm_narrow.h); b_kn: B is W (K, Kd, Nd) as the layer stores it,
+// not (K, Nd, Kd).
+template <typename T>
+static int gather_narrow(const T* A, int64_t n_src, const TiledSrc& src, const int32_t* rows, const T* B, int b_kn,
+                         T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd, hipStream_t stream) {
+  launch_narrow<T>(A, n_src, src, rows, B, b_kn, out, epi, n_dst, K, Kd, Nd, stream);
+  ST_CHECK_LAUNCH();
+  return ST_OK;
+}
+
 template <typename T, typename Src>
 static int launch_gather(const T* A, int64_t n_src, const Src& src, const uint32_t* masks, int W,
                          const int32_t* rows, const T* Bt, T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd,
@@ -2117,8 +2129,13 @@ int ops_gather_map(const T* A, int64_t n_src, const int32_t* map, int64_t ks, in
 template <typename T>
 int ops_gather_tiled(const T* A, int64_t n_src, const int32_t* perm, const int32_t* nk, const int16_t* klist,
                      const int32_t* tmap, const T* Bt, T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd,
-                     hipStream_t stream, int rev) {
+                     hipStream_t stream, int rev, int b_kn) {
   TiledSrc src{nk, klist, tmap, K, rev};
+  if constexpr (sizeof(T) == 2) {
+    if (narrow_ok(n_src, n_dst, K, Kd, Nd, sizeof(T), false, A))
+      return gather_narrow<T>(A, n_src, src, perm, Bt, b_kn, out, epi, n_dst, K, Kd, Nd, stream);
+  }
+  if (b_kn) return ST_ERR_UNSUPPORTED;
   return launch_gather<T>(A, n_src, src, nullptr, (K + 31) / 32, perm, Bt, out, epi, n_dst, K, Kd, Nd, stream);
 }
 
@@ -2222,5 +2239,5 @@ int ops_weight_prep(const T* w, T* out, int K, int Cin, int Cout, int mode, hipS
                                    const int32_t*, int, const T*, T*, const T*, int, int, hipStream_t);             \
   X template int ops_gather_tiled<T>(const T*, int64_t, const int32_t*, const int32_t*, const int16_t*,              \
                                      const int32_t*, const T*, T*, Epi<T>, int64_t, int, int, int, hipStream_t,    \
-                                     int);                                                                         \
+                                     int, int);                                                                    \
   }

@@ -66,17 +66,25 @@ def tiled_ok(dtype: torch.dtype, Kd: int) -> bool:
 
 
 def gather_gemm_tiled(A: torch.Tensor, tiles, Bt: torch.Tensor, n_dst: int, K: int, bias=None,
-                      reverse_k: bool = False) -> torch.Tensor:
+                      reverse_k: bool = False, b_kn: bool = False) -> torch.Tensor:
     """out[perm[t]] = sum over the tile's offsets of A[source] @ Bt[k]^T (+ bias), over a tile plan;
-    with ``reverse_k`` offset k's sources meet Bt[K - 1 - k]."""
+    with ``reverse_k`` offset k's sources meet Bt[K - 1 - k]; with ``b_kn`` (where ``b_kn_ok``) Bt is
+    W (K, C_in, C_out) as the layer stores it."""
     Kd = A.shape[1]
-    Nd = Bt.shape[1]
+    Nd = Bt.shape[2 if b_kn else 1]
     out = torch.empty((n_dst, Nd), dtype=A.dtype, device=A.device)
     _lib.call("st_gather_gemm_tiled", _lib.ptr(A), A.shape[0], tiles.perm_ptr, tiles.nk_ptr,
               tiles.klist_ptr, tiles.tmap_ptr, _lib.ptr(Bt), _lib.ptr(bias), _lib.ptr(out), n_dst, K,
-              Kd, Nd, _lib.compute_code(A.dtype), _lib.GATHER_REVERSE_K if reverse_k else 0,
+              Kd, Nd, _lib.compute_code(A.dtype),
+              (_lib.GATHER_REVERSE_K if reverse_k else 0) | (_lib.GATHER_B_KN if b_kn else 0),
               _lib.stream_of(A.device))
     return out
+
+
+def b_kn_ok(A: torch.Tensor, n_dst: int, K: int, Nd: int) -> bool:
+    """Whether the tiled gather-GEMM reads W (K, C_in, C_out) itself (no transposed copy)."""
+    return _lib.lib().st_gather_b_kn_ok(_lib.ptr(A), A.shape[0], n_dst, K, A.shape[1], Nd,
+                                        _lib.compute_code(A.dtype)) == 1
 
 
 def gather_gemm_fwd(A: torch.Tensor, kmap: KernelMap, Bt: torch.Tensor, bias=None) -> torch.Tensor:
@@ -87,6 +95,14 @@ def gather_gemm_fwd(A: torch.Tensor, kmap: KernelMap, Bt: torch.Tensor, bias=Non
     plan = kmap.forward_plan()
     return gather_gemm(A, kmap.nbr, kmap.k_stride, kmap.r_stride, kmap.out_masks, Bt, kmap.n_out, kmap.K,
                        rows=plan.perm, bias=bias)
+
+
+def conv_forward(A: torch.Tensor, kmap: KernelMap, W: torch.Tensor, bias=None) -> torch.Tensor:
+    """``gather_gemm_fwd`` with the layer's weights W (K, C_in, C_out), transposed first where the
+    kernel does not read them as they are."""
+    if b_kn_ok(A, kmap.n_out, kmap.K, W.shape[2]):
+        return gather_gemm_tiled(A, kmap.forward_tiles(), W, kmap.n_out, kmap.K, bias=bias, b_kn=True)
+    return gather_gemm_fwd(A, kmap, weight_prep(W, _lib.W_TRANSPOSE), bias=bias)
 
 
 def conv_forward_epilogue(features: torch.Tensor, weights: torch.Tensor, kmap: KernelMap, bias, scale, shift,
@@ -295,12 +311,11 @@ class ConvPrecomputedNeighborGEMM(torch.autograd.Function):
         assert kmap.K == K, f"kernel map has {kmap.K} offsets, weights {K}"
         features = features.contiguous()
         w = weights.to(features.dtype).contiguous()
-        wt = weight_prep(w, _lib.W_TRANSPOSE)
         b = None
         if bias is not None:
             assert bias.shape == (C_out,), f"bias must have shape ({C_out},), got {tuple(bias.shape)}"
             b = bias.to(features.dtype).contiguous()
-        out = gather_gemm_fwd(features, kmap, wt, bias=b)
+        out = conv_forward(features, kmap, w, bias=b)
         ctx.save_for_backward(features, weights)
         ctx.kmap = kmap
         ctx.bias_dtype = None if bias is None else bias.dtype

@@ -1,5 +1,6 @@
 """Kernels of the layers with few channels, on random maps, against the float64 oracle: the fp32
-weight gradient with whole-row loads (implicit_precomputed_gemm.py:180-230)."""
+weight gradient with whole-row loads (implicit_precomputed_gemm.py:180-230) and the gather-GEMM that keeps its
+weights in LDS (implicit_precomputed_gemm.py:64-177)."""
 import numpy as np
 import pytest
 import torch
@@ -60,3 +61,99 @@ def test_f32_weight_gradient_rows_non_finite(device):
                torch.float32).cpu().numpy()
     assert np.isfinite(dW[[0, 2]]).all() and np.isfinite(np.delete(dW[1], 5, axis=0)).all()
     assert not np.isfinite(dW[1, 5]).any()
+
+
+def _tiled(nbr, n_in, device):
+    """The tile plan of a (n_out, K) map, rows in the mask-sorted order."""
+    from sparsetriton_amd.nn.functional.conv.kmap import TileMap, TilePlan
+    n_out, K = nbr.shape
+    W = (K + 31) // 32
+    bits = np.zeros((n_out, W * 32), dtype=np.uint64)
+    bits[:, :K] = nbr >= 0
+    masks = (bits.reshape(n_out, W, 32) << np.arange(32, dtype=np.uint64)).sum(2).astype(np.uint32)
+    m = torch.as_tensor(masks.view(np.int32), device=device)
+    nbr_t = torch.as_tensor(np.ascontiguousarray(nbr.T), device=device)
+    perm = TilePlan.build(n_out, K, m).perm
+    return TileMap.build(nbr_t, n_out, 1, m, K, perm, n_out, n_in)
+
+
+EPS = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}  # unit roundoffs (24, 8, 11 bits)
+GATHER = [
+    # n_out, n_in, K, Kd, Nd, density
+    (1, 3, 27, 4, 16, 1.0), (15, 20, 27, 16, 16, 0.5), (17, 20, 27, 32, 32, 0.2), (127, 90, 27, 8, 20, 0.3),
+    (129, 200, 27, 16, 32, 0.9), (1000, 1300, 27, 20, 32, 0.15), (5000, 4000, 27, 12, 3, 0.2), (5000, 4000, 27, 32, 20, 0.2),
+    (3000, 3000, 1, 32, 64, 0.9), (3000, 3000, 8, 64, 32, 0.3), (3000, 3000, 27, 64, 16, 0.1), (2000, 2500, 64, 16, 16, 0.1),
+    (2000, 2500, 27, 16, 64, 0.2), (2000, 2500, 3, 24, 48, 0.4), (700, 700, 27, 40, 16, 0.3), (4000, 3000, 27, 32, 32, 0.0),
+    (70000, 70000, 27, 16, 16, 0.1), (40000, 40000, 27, 4, 32, 0.2),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n_out,n_in,K,Kd,Nd,density", GATHER)
+def test_narrow_gather(device, dtype, n_out, n_in, K, Kd, Nd, density):
+    """The LDS-resident-weights gather-GEMM: row counts around its 16-row wave tiles and the plan's
+    128-row tiles, offset counts, widths with padding on either side, both weight layouts (bitwise
+    equal) and reversed offsets.  A sum of m exact products accumulated in fp32 and rounded once is off
+    by at most (m + 2) 2^-24 of the sum of magnitudes and half a unit of the result; a split fp32
+    product by 2^-15 of its magnitude."""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import b_kn_ok, gather_gemm_tiled
+    rng = np.random.default_rng(n_out + 31 * K + Kd + 7 * Nd)
+    nbr = _map(rng, n_out, n_in, K, density)
+    X = torch.as_tensor(rng.standard_normal((n_in, Kd)), device=device).to(dtype)
+    W = torch.as_tensor(rng.standard_normal((K, Kd, Nd)), device=device).to(dtype)
+    b = torch.as_tensor(rng.standard_normal(Nd), device=device).to(dtype)
+    tiles = _tiled(nbr, n_in, device)
+    if not b_kn_ok(X, n_out, K, Nd):  # (fp32: twice the LDS)
+        assert dtype == torch.float32 and Kd > 16 and Nd >= 32
+        pytest.skip("not built for fp32")
+    y = gather_gemm_tiled(X, tiles, W, n_out, K, bias=b, b_kn=True)
+    yt = gather_gemm_tiled(X, tiles, W.transpose(1, 2).contiguous(), n_out, K, bias=b)
+    assert torch.equal(y, yt)
+    yr = gather_gemm_tiled(X, tiles, W.flip(0).contiguous(), n_out, K, bias=b, reverse_k=True, b_kn=True)
+    assert torch.equal(y, yr)
+    Xd, Wd, bd = X.double().cpu().numpy(), W.double().cpu().numpy(), b.double().cpu().numpy()
+    ref = O.fwd_f64_blas(Xd, Wd, nbr) + bd
+    mag = O.fwd_f64_blas(np.abs(Xd), np.abs(Wd), nbr) + np.abs(bd)
+    m = int((nbr >= 0).sum(1).max()) * Kd
+    bound = ((m + 2) * 2.0 ** -24 + (2.0 ** -15 if dtype == torch.float32 else 0)) * mag + EPS[dtype] * np.abs(ref)
+    assert np.all(np.abs(y.double().cpu().numpy() - ref) <= bound * 1.001 + 1e-30)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Kd,Nd", [(4, 16), (16, 20), (32, 32)])
+def test_narrow_gather_takes_views_and_contains_non_finite_rows(device, dtype, Kd, Nd):
+    """Rows that start 8 bytes (16-bit) into an allocation give the aligned rows' result; a source row
+    with inf reaches only the outputs that pair it."""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import gather_gemm_tiled
+    rng = np.random.default_rng(Kd + Nd)
+    n = n_in = 900
+    K = 27
+    nbr = _map(rng, n, n, K, 0.2)
+    tiles = _tiled(nbr, n_in, device)
+    X = torch.as_tensor(rng.standard_normal((n, Kd)), device=device).to(dtype)
+    W = torch.as_tensor(rng.standard_normal((K, Kd, Nd)), device=device).to(dtype)
+    y = gather_gemm_tiled(X, tiles, W, n, K, b_kn=True)
+    buf = torch.zeros(n * Kd + 4, dtype=dtype, device=device)
+    view = buf[4:].view(n, Kd)
+    view.copy_(X)
+    yv = gather_gemm_tiled(view, tiles, W.transpose(1, 2).contiguous(), n, K)
+    assert torch.allclose(y.float(), yv.float(), rtol=2 * EPS[dtype], atol=1e-5)
+    X[17, 1] = float("inf")
+    hit = (nbr == 17).any(1)
+    y2 = gather_gemm_tiled(X, tiles, W, n, K, b_kn=True)
+    assert torch.equal(torch.isfinite(y2).all(1).cpu(), torch.as_tensor(~hit))
+    assert torch.equal(y2[torch.as_tensor(~hit)], y[torch.as_tensor(~hit)])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("kw", [dict(Kd=6, Nd=16), dict(Kd=128, Nd=16), dict(Kd=16, Nd=65), dict(K=65), dict(Kd=64, Nd=64),
+                                dict(Kd=32, n=262145), dict(Kd=64, n=131073)])
+def test_narrow_gather_refuses_other_shapes(device, dtype, kw):
+    """Host rule: shapes outside the kernel's ranges go to the other kernels."""
+    from sparsetriton_amd import _lib
+    a = {"K": 27, "Kd": 16, "Nd": 16, "n": 100}
+    a.update(kw)
+    args = (None, a["n"], a["n"], a["K"], a["Kd"], a["Nd"], _lib.compute_code(dtype))
+    assert _lib.lib().st_gather_b_kn_ok(*args) == 0
+    assert _lib.lib().st_gather_b_kn_ok(None, 100, 100, 27, 16, 16, _lib.compute_code(dtype)) == 1
+    assert _lib.lib().st_gather_b_kn_ok(None, 1 << 27, 100, 27, 16, 16, _lib.compute_code(dtype)) == 0
