@@ -579,6 +579,19 @@ int st_gather_gemm_tiled_epilogue(const void* A, int64_t n_src, const int32_t* p
                                   st_stream_t stream);
 
 /*
+ * st_gather_gemm_tiled_epilogue with the batch norm given as the layer keeps it
+ * (norm.py:105-112, evaluation mode): scale = bn_weight / sqrt(bn_var + eps)
+ * and shift = bn_bias - bn_mean * scale are formed per column inside the
+ * kernel.  bn_* fp32 (Nd); bn_weight / bn_bias NULL: 1 / 0.  flags: 0 or
+ * ST_GATHER_B_KN.
+ */
+int st_gather_gemm_tiled_bn(const void* A, int64_t n_src, const int32_t* perm, const int32_t* tile_nk,
+                            const int16_t* tile_klist, const int32_t* tile_map, const void* Bt, const void* bias,
+                            const float* bn_weight, const float* bn_bias, const float* bn_mean, const float* bn_var,
+                            float eps, const void* residual, int relu, void* out, int64_t n_dst, int K, int Kd, int Nd,
+                            int dtype, int flags, st_stream_t stream);
+
+/*
  * Weight gradient of ConvPrecomputedNeighborGEMM (precomputed_bwd_weight_kernel,
  * implicit_precomputed_gemm.py:180-230) over the map itself:
  *   dW[k] = sum over o with map(k, o) >= 0 of X[map(k, o)]^T @ dY[o]

@@ -103,6 +103,8 @@ _SIGNATURES = {
     "st_gather_b_kn_ok": [_P, _L, _L, _I, _I, _I, _I],
     "st_gather_gemm_tiled_epilogue": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _P, _L, _I, _I, _I, _I,
                                       _P],
+    "st_gather_gemm_tiled_bn": [_P, _L, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, ctypes.c_float, _P, _I, _P, _L, _I, _I,
+                                _I, _I, _I, _P],
     "st_gather_gemm": [_P, _L, _P, _L, _L, _P, _I, _P, _P, _P, _P, _L, _I, _I, _I, _I, _P],
     "st_wgrad": [_P, _L, _P, _P, _L, _L, _P, _L, _I, _I, _I, _I, _P, _L, _P, _I, _P],
     "st_hashfly_gemm": [_P, _L, _P, _I, _L, _P, ctypes.POINTER(Lookup), _P, _P, _L, _P, _P, _P, _I, _I, _I, _P],

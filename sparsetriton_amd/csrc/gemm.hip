@@ -307,29 +307,50 @@ int st_gather_b_kn_ok(const void* A, int64_t n_src, int64_t n_dst, int K, int Kd
   return narrow_ok(n_src, n_dst, K, Kd, Nd, x3 ? 4 : 2, x3, A) ? 1 : 0;
 }
 
+// Both store-epilogue entry points: the batch norm folded (scale, shift) or as its running statistics (mean, var, eps).
+static int gather_tiled_epi(const void* A, int64_t n_src, const int32_t* perm, const int32_t* tile_nk,
+                            const int16_t* tile_klist, const int32_t* tile_map, const void* Bt, const void* bias,
+                            const float* scale, const float* shift, const float* mean, const float* var, float eps,
+                            const void* residual, int relu, void* out, int64_t n_dst, int K, int Kd, int Nd, int dtype,
+                            int flags, st_stream_t stream) {
+  if (n_src < 0 || n_dst < 0 || K <= 0 || K > ST_MAX_KVOL || Kd <= 0 || Nd <= 0) return ST_ERR_ARG;
+  if (flags & ~ST_GATHER_B_KN) return ST_ERR_ARG;
+  if (n_dst >= (1ll << 31) || n_src >= (1ll << 31)) return ST_ERR_ARG;
+  if (n_dst == 0) return ST_OK;
+  if (!perm || !tile_nk || !tile_klist || !tile_map || !Bt || !out || (n_src > 0 && !A)) return ST_ERR_ARG;
+  const int kn = (flags & ST_GATHER_B_KN) ? 1 : 0;
+  if (dtype == ST_F32_BF16X3) {
+    const Epi<float> epi{(const float*)bias, scale, shift, (const float*)residual, relu ? 1 : 0, mean, var, eps};
+    if (n_src == 0) return fill_output_epi<float>(out, n_dst, Nd, epi, stream);
+    return ops_gather_tiled_x3((const float*)A, n_src, perm, tile_nk, tile_klist, tile_map, (const float*)Bt,
+                               (float*)out, epi, n_dst, K, Kd, Nd, stream, 0, kn);
+  }
+#define ST_EPI(T) Epi<T>{(const T*)bias, scale, shift, (const T*)residual, relu ? 1 : 0, mean, var, eps}
+  ST_DISPATCH_DTYPE(dtype, T, (n_src == 0) ? fill_output_epi<T>(out, n_dst, Nd, ST_EPI(T), stream)
+                                           : ops_gather_tiled<T>((const T*)A, n_src, perm, tile_nk, tile_klist, tile_map,
+                                                                 (const T*)Bt, (T*)out, ST_EPI(T), n_dst, K, Kd, Nd,
+                                                                 stream, 0, kn));
+#undef ST_EPI
+}
+
 int st_gather_gemm_tiled_epilogue(const void* A, int64_t n_src, const int32_t* perm, const int32_t* tile_nk,
                                   const int16_t* tile_klist, const int32_t* tile_map, const void* Bt,
                                   const void* bias, const float* scale, const float* shift, const void* residual,
                                   int relu, void* out, int64_t n_dst, int K, int Kd, int Nd, int dtype,
                                   st_stream_t stream) {
-  if (n_src < 0 || n_dst < 0 || K <= 0 || K > ST_MAX_KVOL || Kd <= 0 || Nd <= 0) return ST_ERR_ARG;
-  if (n_dst >= (1ll << 31) || n_src >= (1ll << 31)) return ST_ERR_ARG;
-  if (n_dst == 0) return ST_OK;
-  if (!perm || !tile_nk || !tile_klist || !tile_map || !Bt || !out || (n_src > 0 && !A)) return ST_ERR_ARG;
   if (shift && !scale) return ST_ERR_ARG;
-  if (dtype == ST_F32_BF16X3) {
-    const Epi<float> epi{(const float*)bias, scale, shift, (const float*)residual, relu ? 1 : 0};
-    if (n_src == 0) return fill_output_epi<float>(out, n_dst, Nd, epi, stream);
-    return ops_gather_tiled_x3((const float*)A, n_src, perm, tile_nk, tile_klist, tile_map, (const float*)Bt,
-                               (float*)out, epi, n_dst, K, Kd, Nd, stream, 0, 0);
-  }
-  ST_DISPATCH_DTYPE(dtype, T, (n_src == 0)
-                                  ? fill_output_epi<T>(out, n_dst, Nd, Epi<T>{(const T*)bias, scale, shift, (const T*)residual, relu ? 1 : 0},
-                                                       stream)
-                                  : ops_gather_tiled<T>((const T*)A, n_src, perm, tile_nk, tile_klist, tile_map,
-                                                        (const T*)Bt, (T*)out,
-                                                        Epi<T>{(const T*)bias, scale, shift, (const T*)residual, relu ? 1 : 0}, n_dst, K,
-                                                        Kd, Nd, stream, 0, 0));
+  return gather_tiled_epi(A, n_src, perm, tile_nk, tile_klist, tile_map, Bt, bias, scale, shift, nullptr, nullptr, 0.f,
+                          residual, relu, out, n_dst, K, Kd, Nd, dtype, 0, stream);
+}
+
+int st_gather_gemm_tiled_bn(const void* A, int64_t n_src, const int32_t* perm, const int32_t* tile_nk,
+                            const int16_t* tile_klist, const int32_t* tile_map, const void* Bt, const void* bias,
+                            const float* bn_weight, const float* bn_bias, const float* bn_mean, const float* bn_var,
+                            float eps, const void* residual, int relu, void* out, int64_t n_dst, int K, int Kd, int Nd,
+                            int dtype, int flags, st_stream_t stream) {
+  if (!bn_mean || !bn_var) return ST_ERR_ARG;
+  return gather_tiled_epi(A, n_src, perm, tile_nk, tile_klist, tile_map, Bt, bias, bn_weight, bn_bias, bn_mean, bn_var,
+                          eps, residual, relu, out, n_dst, K, Kd, Nd, dtype, flags, stream);
 }
 
 int st_wgrad(const void* X, int64_t n_in, const void* dY, const int32_t* map, int64_t map_k_stride,

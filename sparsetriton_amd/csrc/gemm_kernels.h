@@ -1696,7 +1696,7 @@ template <typename T, typename Src>
 static int launch_gather(const T* A, int64_t n_src, const Src& src, const uint32_t* masks, int W,
                          const int32_t* rows, const T* Bt, T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd,
                          hipStream_t stream) {
-  if (epi.scale || epi.shift || epi.residual || epi.relu) {
+  if (epi.scale || epi.shift || epi.var || epi.residual || epi.relu) {
     if constexpr (Src::kTiled)
       return launch_gather_e<T, Src, Epi<T>>(A, n_src, src, masks, W, rows, Bt, out, epi, n_dst, K, Kd, Nd, stream);
     else

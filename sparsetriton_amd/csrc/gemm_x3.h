@@ -813,7 +813,7 @@ template <typename Src>
 static int launch_gather_x3(const float* A, int64_t n_src, const Src& src, const uint32_t* masks, int W,
                             const int32_t* rows, const float* Bt, float* out, Epi<float> epi, int64_t n_dst, int K,
                             int Kd, int Nd, hipStream_t stream) {
-  if (epi.scale || epi.shift || epi.residual || epi.relu) {
+  if (epi.scale || epi.shift || epi.var || epi.residual || epi.relu) {
     if constexpr (Src::kTiled)
       return launch_gather_x3_e<Src, Epi<float>>(A, n_src, src, masks, W, rows, Bt, out, epi, n_dst, K, Kd, Nd,
                                                  stream);

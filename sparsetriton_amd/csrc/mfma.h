@@ -154,12 +154,15 @@ __device__ __forceinline__ T from_f32(float v) {
 }
 
 // Store epilogue of the gather-GEMMs, on the fp32 accumulator of (row r, column c):
-//   v = (acc + bias[c]) * scale[c] + shift[c] + residual[r, c], then ReLU when relu is set
+//   v = (acc + bias[c]) * mul[c] + add[c] + residual[r, c], then ReLU when relu is set
 // bias (the convolution's, conv.py:227-228) and residual (n_dst x Nd, rows in
 // output order: a residual block's shortcut, blocks.py:121-124) have the
-// output dtype; scale and shift are fp32 (an evaluation-mode batch norm folded
-// to one affine map per channel, nn/functional/norm.py:105-112).  A null
-// pointer drops its term.
+// output dtype.  The affine map per channel is an evaluation-mode batch norm
+// (nn/functional/norm.py:105-112), all fp32: given folded, mul = scale and
+// add = shift; or, with var, from its running statistics as the layer keeps
+// them, mul = scale / sqrt(var + eps), add = shift - mean * mul -- every
+// workgroup folds its columns in a few instructions, where a fold on the host's
+// side was six launches per layer.  A null pointer drops its term.
 template <typename T>
 struct Epi {
   static constexpr bool kReads = true;  // reads memory per element (the residual)
@@ -168,18 +171,24 @@ struct Epi {
   const float* shift;
   const T* residual;
   int relu;
+  const float* mean = nullptr;
+  const float* var = nullptr;
+  float eps = 0.f;
   __device__ __forceinline__ void column(int col, int Nd, float& mul, float& add) const {
     const float b = (bias && col < Nd) ? (float)bias[col] : 0.f;
-    if (scale && col < Nd) {
+    mul = 1.f;
+    add = b;
+    if (col >= Nd) return;
+    if (var) {
+      mul = rsqrtf(var[col] + eps) * (scale ? scale[col] : 1.f);
+      add = b * mul + ((shift ? shift[col] : 0.f) - mean[col] * mul);
+    } else if (scale) {
       mul = scale[col];
       add = b * mul + (shift ? shift[col] : 0.f);
-    } else {
-      mul = 1.f;
-      add = b;
     }
   }
   __device__ __forceinline__ float apply(float acc, float mul, float add, int64_t row, int Nd, int col) const {
-    float v = scale ? fmaf(acc, mul, add) : acc + add;
+    float v = (scale || var) ? fmaf(acc, mul, add) : acc + add;
     if (residual) v += (float)residual[row * Nd + col];
     return (relu && v < 0.f) ? 0.f : v;  // (a NaN stays NaN, as under torch.relu)
   }

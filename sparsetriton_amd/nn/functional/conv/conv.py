@@ -114,17 +114,19 @@ def sparse_conv3d_fused(
     shift: torch.Tensor = None,
     residual: torch.Tensor = None,
     relu: bool = False,
+    bn: tuple = None,
 ) -> SparseTensor:
     """Inference convolution with ``act((conv + bias) * scale + shift + residual)`` applied as the
-    GEMM stores its rows (an evaluation-mode conv / batch norm / ReLU block in one pass).  Needs the
-    precomputed-map algorithm and no autograd."""
+    GEMM stores its rows (an evaluation-mode conv / batch norm / ReLU block in one pass); ``bn`` =
+    (weight, bias, running_mean, running_var, eps) gives the batch norm unfolded instead of
+    ``scale`` and ``shift``.  Needs the precomputed-map algorithm and no autograd."""
     if get_conv_algo() != ConvAlgo.PrecomputedNeighborGEMM:
         raise ValueError("the fused epilogue runs on the precomputed-map algorithm")
     if torch.is_grad_enabled() and (tensor.F.requires_grad or weight.requires_grad or
                                     (bias is not None and bias.requires_grad)):
         raise ValueError("the fused epilogue is an inference path (no autograd); call it under torch.no_grad()")
     return _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding, transposed, submanifold,
-                          epilogue=(scale, shift, residual, relu))
+                          epilogue=(scale, shift, residual, relu, bn))
 
 
 def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding, transposed, submanifold,

@@ -105,11 +105,16 @@ def conv_forward(A: torch.Tensor, kmap: KernelMap, W: torch.Tensor, bias=None) -
     return gather_gemm_fwd(A, kmap, weight_prep(W, _lib.W_TRANSPOSE), bias=bias)
 
 
+def _f32(t):
+    return None if t is None else t.detach().to(torch.float32).contiguous()
+
+
 def conv_forward_epilogue(features: torch.Tensor, weights: torch.Tensor, kmap: KernelMap, bias, scale, shift,
-                          residual, relu: bool) -> torch.Tensor:
+                          residual, relu: bool, bn=None) -> torch.Tensor:
     """Forward with the store epilogue ``act((sum + bias) * scale + shift + residual)`` (inference:
-    no autograd).  ``scale`` / ``shift`` fp32 (C_out) or None; ``bias`` and ``residual`` (N_out, C_out)
-    in the features' dtype, residual rows in output order."""
+    no autograd).  ``scale`` / ``shift`` fp32 (C_out) or None; ``bn`` = (weight, bias, running_mean,
+    running_var, eps) instead folds an evaluation-mode batch norm inside the kernel; ``bias`` and
+    ``residual`` (N_out, C_out) in the features' dtype, residual rows in output order."""
     _lib.require_device(features, "features")
     N_in, C_in = features.shape
     K, C_in_w, C_out = weights.shape
@@ -118,20 +123,30 @@ def conv_forward_epilogue(features: torch.Tensor, weights: torch.Tensor, kmap: K
     if not tiled_ok(features.dtype, C_in):
         raise ValueError(f"the fused-epilogue forward covers reduction widths up to the tiled kernels' ({C_in})")
     A = features.contiguous()
-    wt = weight_prep(weights.to(A.dtype).contiguous(), _lib.W_TRANSPOSE)
+    w = weights.to(A.dtype).contiguous()
     b = None if bias is None else bias.detach().to(A.dtype).contiguous()
-    sc = None if scale is None else scale.detach().to(torch.float32).contiguous()
-    sh = None if shift is None else shift.detach().to(torch.float32).contiguous()
     res = None
     if residual is not None:
         assert residual.shape == (kmap.n_out, C_out), "residual must be (N_out, C_out)"
         res = residual.detach().to(A.dtype).contiguous()
     tiles = kmap.forward_tiles()
     out = torch.empty((kmap.n_out, C_out), dtype=A.dtype, device=A.device)
-    _lib.call("st_gather_gemm_tiled_epilogue", _lib.ptr(A), N_in, tiles.perm_ptr, tiles.nk_ptr,
-              tiles.klist_ptr, tiles.tmap_ptr, _lib.ptr(wt), _lib.ptr(b), _lib.ptr(sc), _lib.ptr(sh),
-              _lib.ptr(res), int(bool(relu)), _lib.ptr(out), kmap.n_out, K, C_in, C_out,
-              _lib.compute_code(A.dtype), _lib.stream_of(A.device))
+    plan = (_lib.ptr(A), N_in, tiles.perm_ptr, tiles.nk_ptr, tiles.klist_ptr, tiles.tmap_ptr)
+    dims = (kmap.n_out, K, C_in, C_out, _lib.compute_code(A.dtype))
+    stream = _lib.stream_of(A.device)
+    if bn is not None:
+        kn = b_kn_ok(A, kmap.n_out, K, C_out)
+        if not kn:
+            w = weight_prep(w, _lib.W_TRANSPOSE)
+        bw, bb, mean, var = (_f32(t) for t in bn[:4])
+        _lib.call("st_gather_gemm_tiled_bn", *plan, _lib.ptr(w), _lib.ptr(b), _lib.ptr(bw), _lib.ptr(bb),
+                  _lib.ptr(mean), _lib.ptr(var), float(bn[4]), _lib.ptr(res), int(bool(relu)), _lib.ptr(out), *dims,
+                  _lib.GATHER_B_KN if kn else 0, stream)
+        return out
+    w = weight_prep(w, _lib.W_TRANSPOSE)
+    sc, sh = _f32(scale), _f32(shift)
+    _lib.call("st_gather_gemm_tiled_epilogue", *plan, _lib.ptr(w), _lib.ptr(b), _lib.ptr(sc), _lib.ptr(sh),
+              _lib.ptr(res), int(bool(relu)), _lib.ptr(out), *dims, stream)
     return out
 
 

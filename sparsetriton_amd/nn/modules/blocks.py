@@ -52,8 +52,7 @@ class _ConvBnReLU(nn.Sequential):
     def forward(self, x: SparseTensor) -> SparseTensor:
         if len(self) == 3 and _fusable(self[1], self[2]):
             if _store_fusable(self[0], self[1], x):
-                scale, shift = self[1].folded()
-                return self[0].forward_fused(x, scale, shift, relu=True)
+                return self[0].forward_fused(x, relu=True, bn=self[1].running_affine())
             return self[1].forward_act(self[0](x), relu=True)
         return super().forward(x)
 
@@ -120,15 +119,15 @@ class SparseResBlock(nn.Module):
         m = self.main
         if len(m) == 5 and _fusable(m[1], m[2]) and type(m[4]) is SparseBatchNorm and type(self.relu) is ReLU:
             if self._store_fused_ok(x):
-                h = m[0].forward_fused(x, *m[1].folded(), relu=True)
+                h = m[0].forward_fused(x, relu=True, bn=m[1].running_affine())
                 if isinstance(self.shortcut, nn.Identity):
                     sc = x.F
                 else:
-                    sc = self.shortcut[0].forward_fused(x, *self.shortcut[1].folded()).F
+                    sc = self.shortcut[0].forward_fused(x, bn=self.shortcut[1].running_affine()).F
                 if sc.shape != (h.F.shape[0], m[3].out_channels):
                     raise RuntimeError(f"residual shapes differ: main {(h.F.shape[0], m[3].out_channels)}, "
                                        f"shortcut {tuple(sc.shape)}")
-                return m[3].forward_fused(h, *m[4].folded(), residual=sc.to(h.F.dtype), relu=True)
+                return m[3].forward_fused(h, residual=sc.to(h.F.dtype), relu=True, bn=m[4].running_affine())
             h = m[1].forward_act(m[0](x), relu=True)
             h = m[3](h)
             sc = self.shortcut(x)

@@ -73,13 +73,13 @@ class SparseConv3DBase(nn.Module):
 
 
     def forward_fused(self, input: SparseTensor, scale=None, shift=None, residual=None,
-                      relu: bool = False) -> SparseTensor:
+                      relu: bool = False, bn=None) -> SparseTensor:
         """Inference forward with ``act((conv + bias) * scale + shift + residual)`` fused into the
-        GEMM's store (see ``sparse_conv3d_fused``)."""
+        GEMM's store (see ``sparse_conv3d_fused``); ``bn`` = ``SparseBatchNorm.running_affine()``."""
         return sparse_conv3d_fused(
             input, self.weight, self.kernel_size, bias=self.bias, stride=self.stride, dilation=self.dilation,
             padding=self.padding, transposed=self.transposed, submanifold=self.subm, scale=scale, shift=shift,
-            residual=residual, relu=relu)
+            residual=residual, relu=relu, bn=bn)
 
 
 class SparseConv3D(SparseConv3DBase):

@@ -76,6 +76,10 @@ class SparseBatchNorm(nn.Module):
     def forward(self, input: SparseTensor) -> SparseTensor:
         return self.forward_act(input)
 
+    def running_affine(self):
+        """(weight, bias, running_mean, running_var, eps): the evaluation-mode layer, unfolded."""
+        return self.weight, self.bias, self.running_mean, self.running_var, self.eps
+
     def folded(self):
         """(scale, shift), fp32 (C): evaluation-mode output = input * scale + shift."""
         scale = torch.rsqrt(self.running_var.detach().float() + self.eps)
