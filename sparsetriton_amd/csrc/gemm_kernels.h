@@ -1642,7 +1642,7 @@ static int launch_gather_e(const T* A, int64_t n_src, const Src& src, const uint
   constexpr int VEC = Frag<T>::VEC;
   constexpr int KSTEP = Frag<T>::KSTEP;
   if constexpr (Src::kTiled && sizeof(T) == 2) {
-    if (gather_wide_mode() && wide_ok(Kd, Nd, K, sizeof(T), false, n_src, A, Bt)) {
+    if (gather_wide_mode() && wide_ok(Kd, Nd, K, sizeof(T), false, n_src, n_dst, A, Bt)) {
       launch_wide<T, false, E>(A, n_src, src, rows, Bt, out, epi, n_dst, Kd, Nd, stream);
       ST_CHECK_LAUNCH();
       return ST_OK;

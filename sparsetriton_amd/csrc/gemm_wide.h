@@ -336,10 +336,19 @@ __global__ __launch_bounds__(128 * TP) void gather_gemm_wide_kernel(const T* __r
 // 128 x 128 accumulators that overflows the VGPRs into AGPR copies
 // (SparseResNet21D fp32 step 24.4 -> 39.8 ms with it).  Also: a
 // 3x3x3-sized offset list, 16-byte aligned operands, A and Bt under 2 GB
-// (32-bit buffer offsets).
-inline bool wide_ok(int Kd, int Nd, int K, size_t esz, bool x3, int64_t n_src, const void* A, const void* Bt) {
+// (32-bit buffer offsets).  And enough rows: a wide workgroup covers one or two
+// row tiles and all columns, so a deep stage's few thousand rows leave most CUs
+// idle, where the ring kernels launch two to four times the workgroups (same
+// sums, bit for bit).  Ring / wide, us, indoor voxels (17 pairs a row; a LiDAR
+// set's 4.7 move the crossing up, to over 60,000 rows):
+//   16-bit 128 x 128   9,400 rows 35 / 62   28,700 43 / 64   60,000  75 / 66
+//   fp32    64 x 128   9,400      49 / 85   28,700 61 / 90   60,000 101 / 96
+//   fp32   128 x  64   9,400      88 / 110  28,700 94 / 113  60,000 153 / 127
+inline bool wide_ok(int Kd, int Nd, int K, size_t esz, bool x3, int64_t n_src, int64_t n_dst, const void* A,
+                    const void* Bt) {
   const bool built = (Kd == 64 || Kd == 128) && (Nd == 64 || Nd == 128);
-  const bool faster = x3 ? ((Kd == 128) != (Nd == 128)) : (Kd == 128 && Nd == 128);
+  const bool faster = (x3 ? ((Kd == 128) != (Nd == 128)) : (Kd == 128 && Nd == 128)) &&
+                      n_dst > (x3 && Kd == 128 ? 40960 : 49152);
   return built && (faster || gather_wide_mode() == 2) && K <= kWideMaxK && (uintptr_t)A % 16 == 0 &&
          (uintptr_t)Bt % 16 == 0 && n_src * Kd * (int64_t)esz < (1ll << 31) - 64 &&
          (int64_t)K * Nd * Kd * (int64_t)esz < (1ll << 31) - 64;

@@ -784,7 +784,7 @@ static int launch_gather_x3_e(const float* A, int64_t n_src, const Src& src, con
                               const int32_t* rows, const float* Bt, float* out, E epi, int64_t n_dst, int K, int Kd,
                               int Nd, hipStream_t stream) {
   if constexpr (Src::kTiled) {
-    if (gather_wide_mode() && wide_ok(Kd, Nd, K, sizeof(float), true, n_src, A, Bt)) {
+    if (gather_wide_mode() && wide_ok(Kd, Nd, K, sizeof(float), true, n_src, n_dst, A, Bt)) {
       launch_wide<float, true, E>(A, n_src, src, rows, Bt, out, epi, n_dst, Kd, Nd, stream);
       ST_CHECK_LAUNCH();
       return ST_OK;

@@ -1,0 +1,62 @@
+"""Which gather-GEMM kernel takes a layer, and the batch norm folded in its store."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _layer(device, n, cin, cout, dtype, seed):
+    from sparsetriton_amd import SparseTensor
+    rng = np.random.default_rng(seed)
+    S = max(8, int(round((n / 0.2) ** (1 / 3))))
+    lin = np.sort(rng.choice(S ** 3, n, replace=False))
+    c = np.stack([0 * lin, lin // S ** 2, lin // S % S, lin % S], 1).astype(np.int32)
+    X = torch.as_tensor(rng.standard_normal((n, cin)), device=device).to(dtype)
+    W = torch.as_tensor(rng.standard_normal((27, cin, cout)) / np.sqrt(27 * cin), device=device).to(dtype)
+    sp = SparseTensor(X, torch.as_tensor(c, device=device), spatial_shape=(S, S, S), batch_size=1)
+    nbr = O.exact_kmap(c, c, O.target_offsets(3, 1, 1, False), 1, (S, S, S))
+    return sp, W, nbr, rng
+
+
+@pytest.mark.parametrize("cin,cout,dtype", [(128, 128, torch.bfloat16), (64, 128, torch.float32), (128, 64, torch.float32)])
+@pytest.mark.parametrize("n", [40960, 40961, 49152, 49153])
+def test_wide_and_ring_gathers_meet(device, cin, cout, dtype, n):
+    """The row counts where the wide kernel takes over from the ring kernels: both sides agree with
+    float64 within the rounding of their sums, at the first and the last rows."""
+    from sparsetriton_amd.nn.functional import sparse_conv3d
+    sp, W, nbr, _ = _layer(device, n, cin, cout, dtype, 3)
+    y = sparse_conv3d(sp, W, 3).F
+    rows = np.r_[0:500, n - 500:n]
+    ref = O.fwd_f64_blas(sp.F.double().cpu().numpy(), W.double().cpu().numpy(), nbr[rows])
+    mag = O.fwd_f64_blas(sp.F.double().abs().cpu().numpy(), W.double().abs().cpu().numpy(), nbr[rows])
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -24
+    bound = (27 * cin * 2.0 ** -24 + (2.0 ** -15 if dtype == torch.float32 else 0)) * mag + u * np.abs(ref)
+    assert np.all(np.abs(y[rows].double().cpu().numpy() - ref) <= 1.001 * bound)
+
+
+@pytest.mark.parametrize("cin,cout,dtype", [(16, 16, torch.float32), (32, 20, torch.bfloat16), (64, 64, torch.float16),
+                                            (64, 128, torch.float32), (128, 128, torch.bfloat16)])
+@pytest.mark.parametrize("affine,residual", [(True, True), (False, False), (True, False)])
+def test_batch_norm_folded_in_the_store(device, cin, cout, dtype, affine, residual):
+    """sparse_conv3d_fused with the batch norm's own tensors equals the one folded on the caller's
+    side to the rounding of the fold (two fp32 units of mul and add)."""
+    from sparsetriton_amd.nn.functional import sparse_conv3d_fused
+    sp, W, _, rng = _layer(device, 1500, cin, cout, dtype, cin + cout)
+
+    def vec(lo, hi):
+        return torch.as_tensor(rng.uniform(lo, hi, cout).astype(np.float32), device=device)
+    w, b = (vec(0.5, 1.5), vec(-1, 1)) if affine else (None, None)
+    mean, var, eps = vec(-1, 1), vec(0.01, 2), 1e-5
+    bias = vec(-1, 1).to(dtype)
+    res = torch.as_tensor(rng.standard_normal((1500, cout)), device=device).to(dtype) if residual else None
+    with torch.no_grad():
+        got = sparse_conv3d_fused(sp, W, 3, bias=bias, residual=res, relu=True, bn=(w, b, mean, var, eps)).F
+        scale = torch.rsqrt(var + eps) * (w if affine else 1.0)
+        shift = -mean * scale + (b if affine else 0.0)
+        want = sparse_conv3d_fused(sp, W, 3, bias=bias, scale=scale, shift=shift, residual=res, relu=True).F
+    u = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    tol = 2 * u * want.float().abs() + 8 * 2.0 ** -24 * (want.float().abs() + 40)
+    assert bool(((got.float() - want.float()).abs() <= tol).all())
