@@ -182,7 +182,8 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
                 # brick indexes of the candidates and of the inputs; the hash tables when a box cannot
                 # be indexed or a row's batch index lies outside the tensor's batch count
                 built = brick_out_coords_and_map(tensor.C, tensor.batch_size, tensor.spatial_shape, k, s, d, p,
-                                                 transposed)
+                                                 transposed,
+                                                 with_inverse=torch.is_grad_enabled() and tensor.F.requires_grad)
                 if built is not None:
                     out_coords, new_shape, _, kmap, table_status = built
                 else:

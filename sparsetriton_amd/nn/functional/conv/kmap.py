@@ -839,7 +839,7 @@ def build_out_coords_and_map(in_coords: torch.Tensor, spatial_shape, kernel_size
 
 def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_shape, kernel_size: int,
                              stride: int, dilation: int, padding: int, transposed: bool, with_map: bool = True,
-                             chunk_size: Optional[int] = None):
+                             chunk_size: Optional[int] = None, with_inverse: bool = True):
     """``build_out_coords_and_map`` without hash tables: the same output coordinates in the same
     order and the same map, through brick indexes (``st_outcoords_brick_*`` over the candidates'
     output box, ``st_kmap_strided_query`` over the input coordinates' index).
@@ -848,7 +848,9 @@ def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_s
     (a StatusSnapshot of the input index, or None without a map) carries the bad-coordinate count
     the input hash table would report -- or None when the boxes cannot be indexed or a row's
     batch index lies outside [0, batch_size); the caller then uses ``build_out_coords_and_map``.
-    One host synchronisation reads the output count.
+    ``with_inverse=False`` leaves the transposed map, which only an input gradient reads, to
+    ``KernelMap.ensure_inverse`` (an inference pass never needs it: 71 us of a 240,001 -> 4.3 M row
+    transposed layer's build).  One host synchronisation reads the output count.
     """
     from sparsetriton_amd.utils.hash import StatusSnapshot
 
@@ -907,14 +909,16 @@ def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_s
         return out_coords, torch.Size(new_shape), kernel_offsets, None, None
     W = _mask_words(K)
     nbr = torch.empty((K, n_out), dtype=torch.int32, device=dev)
-    invnbr = torch.empty((K, n), dtype=torch.int32, device=dev)
     out_masks = torch.empty((n_out, W), dtype=torch.int32, device=dev)
-    in_masks = torch.empty((n, W), dtype=torch.int32, device=dev)
     _lib.call("st_kmap_strided_query", _lib.ptr(out_coords), cc, n_out, _lib.ptr(offs), ctypes.byref(g),
               int(batch_size), _lib.ptr(index.work), index.nbytes, n, _lib.ptr(nbr), _lib.ptr(out_masks), s)
-    _lib.call("st_outcoords_brick_inverse", _lib.ptr(in_coords), cc, n, _lib.ptr(offs), ctypes.byref(g),
-              int(batch_size), int(kernel_size), int(dilation), _lib.ptr(work), wbytes, _lib.ptr(index.work),
-              index.nbytes, _lib.ptr(invnbr), _lib.ptr(in_masks), s)
+    invnbr = in_masks = None
+    if with_inverse:
+        invnbr = torch.empty((K, n), dtype=torch.int32, device=dev)
+        in_masks = torch.empty((n, W), dtype=torch.int32, device=dev)
+        _lib.call("st_outcoords_brick_inverse", _lib.ptr(in_coords), cc, n, _lib.ptr(offs), ctypes.byref(g),
+                  int(batch_size), int(kernel_size), int(dilation), _lib.ptr(work), wbytes, _lib.ptr(index.work),
+                  index.nbytes, _lib.ptr(invnbr), _lib.ptr(in_masks), s)
     kmap = KernelMap(nbr, n, n_out, K, out_masks=out_masks, invnbr=invnbr, in_masks=in_masks)
     return out_coords, torch.Size(new_shape), kernel_offsets, kmap, index.status
 

@@ -60,3 +60,28 @@ def test_batch_norm_folded_in_the_store(device, cin, cout, dtype, affine, residu
     u = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
     tol = 2 * u * want.float().abs() + 8 * 2.0 ** -24 * (want.float().abs() + 40)
     assert bool(((got.float() - want.float()).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_transposed_map_after_an_inference_pass(device, transposed):
+    """An inference pass leaves the transposed map out of the cached build; a training pass over the
+    same coordinates builds it then, with the gradients of a build that had it."""
+    from sparsetriton_amd import SparseTensor
+    from sparsetriton_amd.nn.functional import sparse_conv3d
+    sp, _, _, rng = _layer(device, 3000, 16, 16, torch.float32, 9)
+    W = torch.as_tensor(rng.standard_normal((27, 16, 16)).astype(np.float32) / 20, device=device)
+    kw = dict(kernel_size=3, stride=2, padding=1, transposed=transposed, submanifold=False)
+    grads = []
+    for infer_first in (False, True):
+        x = sp.F.clone().requires_grad_(True)
+        w = W.clone().requires_grad_(True)
+        t = SparseTensor(x, sp.C, spatial_shape=sp.spatial_shape, batch_size=1)
+        if infer_first:
+            with torch.no_grad():
+                sparse_conv3d(t, w, **kw)
+            (_, km, _), = t._cache.neighbor_indices.values()
+            assert km.invnbr is None
+        y = sparse_conv3d(t, w, **kw).F
+        g = torch.sin(torch.arange(y.numel(), device=device, dtype=torch.float32)).view_as(y)
+        grads.append(torch.autograd.grad(y, [x, w], g))
+    assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
