@@ -12,6 +12,8 @@ from pathlib import Path
 
 import torch
 
+from sparsetriton_amd.config import get_fp32_precision
+
 _LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libsparsetriton_amd.so"
 
 ST_OK = 0
@@ -221,12 +223,7 @@ F32_BF16X3 = 3
 def compute_code(dtype: torch.dtype) -> int:
     """dtype code for a GEMM entry point: fp32 follows ``config.get_fp32_precision()``."""
     code = feat_code(dtype)
-    if code == 0:
-        from sparsetriton_amd.config import get_fp32_precision
-
-        if get_fp32_precision() == "bf16x3":
-            return F32_BF16X3
-    return code
+    return F32_BF16X3 if code == 0 and get_fp32_precision() == "bf16x3" else code
 
 
 def fill_(t: torch.Tensor, value: int) -> torch.Tensor:

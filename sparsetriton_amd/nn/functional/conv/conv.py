@@ -183,7 +183,8 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
                 # be indexed or a row's batch index lies outside the tensor's batch count
                 built = brick_out_coords_and_map(tensor.C, tensor.batch_size, tensor.spatial_shape, k, s, d, p,
                                                  transposed,
-                                                 with_inverse=torch.is_grad_enabled() and tensor.F.requires_grad)
+                                                 with_inverse=torch.is_grad_enabled() and tensor.F.requires_grad,
+                                                 with_offsets=False)
                 if built is not None:
                     out_coords, new_shape, _, kmap, table_status = built
                 else:
@@ -255,7 +256,7 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
     if submanifold and (out_coords is tensor.C or (out_coords.shape == tensor.C.shape
                                                    and torch.equal(out_coords, tensor.C))):
         return tensor.replace(out_feats)
-    return SparseTensor(feats=out_feats, coords=out_coords, spatial_shape=new_shape, batch_size=tensor.batch_size)
+    return tensor._derive(out_feats, out_coords, new_shape)
 
 
 def _brick_index(tensor: SparseTensor, eligible: bool, K: int, C_in: int, C_out: int):

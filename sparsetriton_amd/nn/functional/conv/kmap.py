@@ -839,7 +839,7 @@ def build_out_coords_and_map(in_coords: torch.Tensor, spatial_shape, kernel_size
 
 def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_shape, kernel_size: int,
                              stride: int, dilation: int, padding: int, transposed: bool, with_map: bool = True,
-                             chunk_size: Optional[int] = None, with_inverse: bool = True):
+                             chunk_size: Optional[int] = None, with_inverse: bool = True, with_offsets: bool = True):
     """``build_out_coords_and_map`` without hash tables: the same output coordinates in the same
     order and the same map, through brick indexes (``st_outcoords_brick_*`` over the candidates'
     output box, ``st_kmap_strided_query`` over the input coordinates' index).
@@ -850,7 +850,7 @@ def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_s
     batch index lies outside [0, batch_size); the caller then uses ``build_out_coords_and_map``.
     ``with_inverse=False`` leaves the transposed map, which only an input gradient reads, to
     ``KernelMap.ensure_inverse`` (an inference pass never needs it: 71 us of a 240,001 -> 4.3 M row
-    transposed layer's build).  One host synchronisation reads the output count.
+    transposed layer's build); ``with_offsets=False`` returns None for the offsets.  One host synchronisation reads the output count.
     """
     from sparsetriton_amd.utils.hash import StatusSnapshot
 
@@ -886,8 +886,9 @@ def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_s
     s = _lib.stream_of(dev)
     cc = _lib.coord_code(in_coords.dtype)
     work = torch.empty((wbytes,), dtype=torch.uint8, device=dev)
-    counts = torch.empty((nblocks + 1,), dtype=torch.int32, device=dev)
-    status = torch.empty((_lib.STATUS_WORDS,), dtype=torch.int32, device=dev)
+    # block counts, the output count, then the status words: the host reads the last two in one copy
+    both = torch.empty((nblocks + 1 + _lib.STATUS_WORDS,), dtype=torch.int32, device=dev)
+    counts, status = both[:nblocks + 1], both[nblocks + 1:]
     offs = _offsets_i32(offsets)
     _lib.call("st_outcoords_brick_plan", _lib.ptr(in_coords), cc, n, _lib.ptr(offs), ctypes.byref(g),
               int(batch_size), int(kernel_size), int(dilation), _lib.ptr(work), wbytes, _lib.ptr(counts), nblocks,
@@ -896,11 +897,11 @@ def brick_out_coords_and_map(in_coords: torch.Tensor, batch_size: int, spatial_s
     if with_map:
         # the input index is queued before the host waits for the output count
         index = BrickIndex.build(in_coords, batch_size, spatial_shape)
-    n_out, outside, over = torch.stack([counts[nblocks], status[_lib.STATUS_OUT_OF_BOX],
-                                        status[_lib.STATUS_OVERFLOW]]).tolist()
-    if outside or over:
+    n_out, *words = both[nblocks:].tolist()
+    if words[_lib.STATUS_OUT_OF_BOX] or words[_lib.STATUS_OVERFLOW]:
         return None
-    kernel_offsets = offsets.to(in_coords.dtype, copy=True)  # returned to the caller: not the shared tensor
+    # returned to the caller: not the shared tensor
+    kernel_offsets = offsets.to(in_coords.dtype, copy=True) if with_offsets else None
     out_coords = torch.empty((n_out, 4), dtype=in_coords.dtype, device=dev)
     _lib.call("st_outcoords_brick_emit", _lib.ptr(in_coords), cc, n, _lib.ptr(offs), ctypes.byref(g),
               int(batch_size), int(kernel_size), int(dilation), _lib.ptr(work), wbytes, _lib.ptr(counts), nblocks,

@@ -18,6 +18,7 @@ features, the residual and the affine parameters.
 """
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -34,10 +35,15 @@ def _f32(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     return t.detach().to(torch.float32).contiguous()
 
 
-def _workspace(n: int, C: int, B: int, device) -> torch.Tensor:
+@functools.lru_cache(maxsize=256)
+def _workspace_floats(n: int, C: int, B: int) -> int:
     floats = ctypes.c_int64()
     _lib.call("st_bn_workspace", n, C, B, ctypes.byref(floats))
-    return torch.empty((floats.value,), dtype=torch.float32, device=device)
+    return floats.value
+
+
+def _workspace(n: int, C: int, B: int, device) -> torch.Tensor:
+    return torch.empty((_workspace_floats(n, C, B),), dtype=torch.float32, device=device)
 
 
 class _BatchNormAct(torch.autograd.Function):
@@ -60,8 +66,7 @@ class _BatchNormAct(torch.autograd.Function):
         out = torch.empty_like(x)
         s = _lib.stream_of(dev)
         if training:
-            mean = torch.empty((B, C), dtype=torch.float32, device=dev)
-            invstd = torch.empty((B, C), dtype=torch.float32, device=dev)
+            mean, invstd = torch.empty((2, B, C), dtype=torch.float32, device=dev).unbind(0)
             counts = torch.empty((B,), dtype=torch.int32, device=dev)
             ws = _workspace(n, C, B, dev)
             rm = rv = None

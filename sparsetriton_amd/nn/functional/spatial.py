@@ -79,7 +79,7 @@ def sparse_pooling(input: SparseTensor, kernel_size: int, padding: int, stride: 
         stride = kernel_size
     new_shape = tuple((int(s) - kernel_size + padding * 2) // stride + 1 for s in input.spatial_shape)
     feats, coords = _Pool.apply(input.F, input.C, kernel_size, padding, stride, mode)
-    return SparseTensor(feats, coords, spatial_shape=new_shape, batch_size=input.batch_size)
+    return input._derive(feats, coords, new_shape)
 
 
 class _Upsample(torch.autograd.Function):
@@ -113,4 +113,4 @@ def sparse_upsample(input: SparseTensor, scale_factor: int = None) -> SparseTens
     _lib.require_device(input.F, "SparseTensor features")
     feats, coords = _Upsample.apply(input.F, input.C, int(scale_factor))
     new_shape = tuple(int(s) * int(scale_factor) for s in input.spatial_shape)
-    return SparseTensor(feats, coords, spatial_shape=new_shape, batch_size=input.batch_size)
+    return input._derive(feats, coords, new_shape)

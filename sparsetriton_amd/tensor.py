@@ -33,6 +33,11 @@ class TensorCache:
         self.neighbor_indices: Dict[Tuple[Any, ...], Tuple[torch.Tensor, Any, Tuple]] = {}
 
 
+def _version(t: torch.Tensor) -> Optional[int]:
+    """The tensor's in-place write count; None under inference mode, which keeps none."""
+    return None if t.is_inference() else t._version
+
+
 class SparseTensor:
     """Sparse 3-D tensor: ``feats`` (N, C) at ``coords`` (N, 4) = (batch, x, y, z)."""
 
@@ -70,8 +75,38 @@ class SparseTensor:
             self.batch_size = batch_size
 
         self._cache = TensorCache() if cache is None else cache
+        self._checked_version = _version(self._coords)
+
+    def _coords_checked(self) -> bool:
+        """Whether the coordinates are the ones the constructor checked: not assigned or written since."""
+        return self._checked_version is not None and self._checked_version == _version(self._coords)
+
+    def _derive(self, feats: torch.Tensor, coords: torch.Tensor, spatial_shape) -> "SparseTensor":
+        """A layer's output on new coordinates whose batch indices are this tensor's.  Where those are
+        still the ones the constructor checked (not assigned or written since), nothing is read back
+        from the device: the constructor's check waits for the stream, which in a training step
+        leaves the GPU idle between the forward and the backward."""
+        if not self._coords_checked():
+            return SparseTensor(feats, coords, spatial_shape=spatial_shape, batch_size=self.batch_size)
+        out = SparseTensor.__new__(SparseTensor)
+        out.feats = feats
+        out.coords = coords.to(device=feats.device, dtype=get_coords_dtype())
+        out.spatial_shape = torch.Size([int(s) for s in spatial_shape])
+        out.batch_size = self.batch_size
+        out._cache = TensorCache()
+        out._checked_version = _version(out._coords)
+        return out
 
     # ------------------------------------------------------------ accessors
+    @property
+    def coords(self) -> torch.Tensor:
+        return self._coords
+
+    @coords.setter
+    def coords(self, coords: torch.Tensor) -> None:
+        self._coords = coords
+        self._checked_version = None  # (see _derive)
+
     @property
     def F(self) -> torch.Tensor:
         return self.feats
@@ -90,8 +125,11 @@ class SparseTensor:
 
     # ------------------------------------------------------------ conversions
     def to(self, device: Union[str, torch.device], non_blocking: bool = False) -> "SparseTensor":
+        checked = self._coords_checked()
         self.feats = self.feats.to(device, non_blocking=non_blocking)
         self.coords = self.coords.to(device, non_blocking=non_blocking)
+        if checked:
+            self._checked_version = _version(self._coords)
         return self
 
     def cpu(self) -> "SparseTensor":
@@ -122,6 +160,8 @@ class SparseTensor:
         out.spatial_shape = self.spatial_shape
         out.batch_size = self.batch_size
         out._cache = self._cache
+        if self._coords_checked():
+            out._checked_version = _version(out._coords)
         return out
 
     def __repr__(self) -> str:

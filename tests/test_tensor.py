@@ -105,3 +105,32 @@ def test_spatial_argument_errors():
         sparse_pooling(sp, kernel_size=2, padding=0, stride=2, mode="invalid")
     with pytest.raises(ValueError, match="mode must be"):
         SparsePooling(kernel_size=2, mode="invalid")
+
+
+def test_derived_tensors_check_coordinates_written_since():
+    """A layer's output skips the constructor's batch check only while its input's coordinates are the
+    ones the constructor checked: assigned, or written in place, they are checked again."""
+    c = torch.tensor([[0, 1, 2, 3], [1, 1, 1, 1]], dtype=torch.int16)
+    f = torch.zeros(2, 4)
+    bad = torch.tensor([[0, 1, 2, 3], [5, 1, 1, 1]], dtype=torch.int16)
+    t = SparseTensor(f, c.clone(), spatial_shape=(8, 8, 8), batch_size=2)
+    out = t.replace(f + 1)._derive(f, c, (4, 4, 4))
+    assert out.batch_size == 2 and tuple(out.spatial_shape) == (4, 4, 4) and out._cache is not t._cache
+    assert out._derive(f, c, (2, 2, 2)).batch_size == 2
+    for how in ("property", "attribute", "in_place"):
+        t = SparseTensor(f, c.clone(), spatial_shape=(8, 8, 8), batch_size=2)
+        if how == "property":
+            t.C = bad
+        elif how == "attribute":
+            t.coords = bad
+        else:
+            t.C[1, 0] = 5
+        for u in (t, t.replace(f), t.to("cpu")):
+            with pytest.raises(AssertionError, match="max batch index"):
+                u._derive(f, u.C, (4, 4, 4))
+    with torch.inference_mode():
+        t = SparseTensor(f.clone(), c.clone(), spatial_shape=(8, 8, 8), batch_size=2)
+        assert t._derive(f, c.clone(), (4, 4, 4)).batch_size == 2
+        t.C[1, 0] = 5
+        with pytest.raises(AssertionError, match="max batch index"):
+            t._derive(f, t.C, (4, 4, 4))
