@@ -1216,13 +1216,14 @@ __global__ __launch_bounds__(256, (MB > 4 || NB > 4) ? 1 : (ONEPASS ? 2 : 3)) vo
   static_assert(Frag<T>::KSTEP == 32 && Frag<T>::VEC == 8, "16-bit MFMA fragments");
   constexpr bool BIG = MB > 4 || NB > 4;
   constexpr bool PREFETCH = ONEPASS || BIG;  // pair indices one step ahead of their rows
+  constexpr bool PIPE = BIG && BUF;          // two stages: rows go to LDS under the previous step's MFMAs
   static_assert(!(ONEPASS && BIG), "a 128-wide tile sums in rounds");
   constexpr int TM = 16 * MB, TN = 16 * NB;
   constexpr int CPRX = TM / 8, RPIX = 64 / CPRX, NVX = 32 / RPIX;
   constexpr int CPRY = TN / 8, RPIY = 64 / CPRY, NVY = 32 / RPIY;
   constexpr int PX = wave_pitch(TM), PY = wave_pitch(TN);
   constexpr int STAGE = 32 * (PX + PY);  // elements per wave (X rows, then dY rows)
-  constexpr int STAGE_BYTES = 4 * STAGE * (int)sizeof(T);
+  constexpr int STAGE_BYTES = (PIPE ? 2 : 1) * 4 * STAGE * (int)sizeof(T);
   constexpr int RP = TN + 4;            // row pitch (floats) of the per-wave tiles summed at the end
   constexpr int RH = (ONEPASS || TM < 32) ? TM : 32;  // rows summed per round
   constexpr int RED_BYTES = 4 * RH * RP * (int)sizeof(float);
@@ -1237,7 +1238,7 @@ __global__ __launch_bounds__(256, (MB > 4 || NB > 4) ? 1 : (ONEPASS ? 2 : 3)) vo
   const int ntn = Cout / TN;
   const ChunkTile ct = chunk_tile(total, (Cin / TM) * ntn);
   const int cm0 = (ct.tile / ntn) * TM, cn0 = (ct.tile % ntn) * TN;
-  T* xs = reinterpret_cast<T*>(lds) + wid * STAGE;
+  T* xs = reinterpret_cast<T*>(lds) + wid * (PIPE ? 2 : 1) * STAGE;
   T* ys = xs + 32 * PX;
   float* red = reinterpret_cast<float*>(lds);
   // loader lanes: lane / CPR is the row within an instruction's RPI rows, lane % CPR its chunk;
@@ -1287,10 +1288,103 @@ __global__ __launch_bounds__(256, (MB > 4 || NB > 4) ? 1 : (ONEPASS ? 2 : 3)) vo
       }
     };
     int q = p0 + wid * 32;
-    int2 prn = load_pairs(q);
-    if (q < p1) load_rows(prn);
-    if constexpr (PREFETCH) prn = load_pairs(q + 128);
-    for (; q < p1; q += 128) {
+    if constexpr (PIPE) {
+      // One wave per SIMD: nothing else runs while it moves rows through LDS, so
+      // the rows of step s + 1 are stored to the other stage, and those of step
+      // s + 2 loaded into the registers this frees, between the MFMAs of step s
+      // (a row block of MFMAs, then its share of the rows).  Steps past the end
+      // move zeros (their loads read nothing).
+      auto store_x = [&](int v, int at) { *reinterpret_cast<F*>(&xs[at + (v * RPIX + lrx) * PX + lcx * 8]) = xr[v]; };
+      auto store_y = [&](int v, int at) { *reinterpret_cast<F*>(&ys[at + (v * RPIY + lry) * PY + lcy * 8]) = yr[v]; };
+      // Pairs of a step as row byte offsets (past the end for a pair past the chunk), one per lane mod 32,
+      // loaded without a branch a step before they are looked at.
+      const int up0 = __builtin_amdgcn_readfirstlane(p0), np = __builtin_amdgcn_readfirstlane(p1) - up0;
+      const __amdgpu_buffer_rsrc_t p_rsrc = make_rsrc(pairs + up0, (int64_t)np * 8);
+      typedef int v2i __attribute__((ext_vector_type(2)));
+      auto load_step = [&](int s) {
+        return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(p_rsrc, (s + (lane & 31)) * 8, 0, 0));
+      };
+      auto row_offsets = [&](v2i pr, int s, int& ox, int& oy) {
+        const bool ok = s + (lane & 31) < np;
+        ox = ok ? (pr[0] * Cin + cm0) * (int)sizeof(T) : kOobOffset;
+        oy = ok ? (pr[1] * Cout + cn0) * (int)sizeof(T) : kOobOffset;
+      };
+      auto load_x = [&](int v, int from) { xr[v] = load16<F>(x_rsrc, (int)((uint32_t)from + lcx * 16)); };
+      auto load_y = [&](int v, int from) { yr[v] = load16<F>(y_rsrc, (int)((uint32_t)from + lcy * 16)); };
+      int s = __builtin_amdgcn_readfirstlane(wid * 32);  // this step's first pair within the chunk
+      v2i pr = load_step(s), prn = load_step(s + 128);
+      int ox, oy;
+      row_offsets(pr, s, ox, oy);
+      // (rows in the loop's order, so that the waits there count the same loads from the first turn on)
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+#pragma unroll
+        for (int v = i * NVX / MB; v < (i + 1) * NVX / MB; ++v) load_x(v, __shfl(ox, v * RPIX + lrx, 64));
+#pragma unroll
+        for (int v = i * NVY / MB; v < (i + 1) * NVY / MB; ++v) load_y(v, __shfl(oy, v * RPIY + lry, 64));
+      }
+      pr = load_step(s + 256);
+      row_offsets(prn, s + 128, ox, oy);
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+#pragma unroll
+        for (int v = i * NVX / MB; v < (i + 1) * NVX / MB; ++v) {
+          store_x(v, 0);
+          load_x(v, __shfl(ox, v * RPIX + lrx, 64));
+        }
+#pragma unroll
+        for (int v = i * NVY / MB; v < (i + 1) * NVY / MB; ++v) {
+          store_y(v, 0);
+          load_y(v, __shfl(oy, v * RPIY + lry, 64));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      int at = 0;
+      for (; s < np; s += 128) {
+        F a[MB], b[NB];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) b[j] = tr_frag<F, T, PY>(ys + at, g, c, j * 16);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) a[i] = tr_frag<F, T, PX>(xs + at, g, c, i * 16);
+        const int next = STAGE - at;
+        row_offsets(pr, s + 256, ox, oy);
+        pr = load_step(s + 384);
+        int fx[NVX], fy[NVY];
+#pragma unroll
+        for (int v = 0; v < NVX; ++v) fx[v] = __shfl(ox, v * RPIX + lrx, 64);
+#pragma unroll
+        for (int v = 0; v < NVY; ++v) fy[v] = __shfl(oy, v * RPIY + lry, 64);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < MB; ++i) {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) acc[i][j] = mfma(a[i], b[j], acc[i][j]);
+#pragma unroll
+          for (int v = i * NVX / MB; v < (i + 1) * NVX / MB; ++v) {
+            store_x(v, next);
+            load_x(v, fx[v]);
+          }
+#pragma unroll
+          for (int v = i * NVY / MB; v < (i + 1) * NVY / MB; ++v) {
+            store_y(v, next);
+            load_y(v, fy[v]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        at = next;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+    int2 prn = make_int2(-1, -1);
+    if constexpr (!PIPE) prn = load_pairs(q);
+    if (!PIPE && q < p1) load_rows(prn);
+    if constexpr (PREFETCH && !PIPE) prn = load_pairs(q + 128);
+    for (; !PIPE && q < p1; q += 128) {
 #pragma unroll
       for (int v = 0; v < (NVX > NVY ? NVX : NVY); ++v) {
         if (v < NVX) *reinterpret_cast<F*>(&xs[(v * RPIX + lrx) * PX + lcx * 8]) = xr[v];
