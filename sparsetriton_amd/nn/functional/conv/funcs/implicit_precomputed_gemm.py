@@ -82,7 +82,11 @@ def gather_gemm_tiled(A: torch.Tensor, tiles, Bt: torch.Tensor, n_dst: int, K: i
 
 
 def b_kn_ok(A: torch.Tensor, n_dst: int, K: int, Nd: int) -> bool:
-    """Whether the tiled gather-GEMM reads W (K, C_in, C_out) itself (no transposed copy)."""
+    """Whether the tiled gather-GEMM reads W (K, C_in, C_out) itself (no transposed copy).  Weights that
+    cannot fit the kernel's 112 KB of LDS need no library call to say so: at 64 -> 64 and 5,000 rows,
+    where the host sets the pace, the call cost 2 of 27 us."""
+    if K * A.shape[1] * Nd * A.element_size() > 112 << 10:
+        return False
     return _lib.lib().st_gather_b_kn_ok(_lib.ptr(A), A.shape[0], n_dst, K, A.shape[1], Nd,
                                         _lib.compute_code(A.dtype)) == 1
 
@@ -301,7 +305,7 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
 def _concurrent_backward(X: torch.Tensor, C_out: int, n_rows: int) -> bool:
     """Whether the weight gradient runs beside the input gradient.  At 16-bit 128 x 128 both run
     one workgroup per CU (the two-tile wide gather, the 128 x 128 per-wave weight gradient), which
-    leaves issue slots the other kernel fills: config 5 step 2.65 -> 2.53 ms.  Elsewhere the kernels
+    leaves issue slots the other kernel fills: 1 M indoor rows, step 2.30 -> 2.26 ms.  Elsewhere the kernels
     already fill the CUs and the cross-stream waits cost more than the overlap gains (config 2 bf16
     0.186 -> 0.21 ms, config 3 / 4 3-8 % slower).  ST_CONCURRENT_BACKWARD=0 / 2 forces it off / on."""
     mode = os.environ.get("ST_CONCURRENT_BACKWARD", "1")
