@@ -67,6 +67,11 @@ inline int64_t narrow_lds(int K, int Kd, int Nd, bool x3) {
 //   fp32   32 x 32   117,000      25.0 / 30.7   160,000 30.6 / 32.2   235,000 36.9 / 33.2
 //   16-bit 64 x 16   117,000      17.5 / 20.2   160,000 20.7 / 21.8   235,000 26.6 / 24.9
 //   16-bit 64 x 32    60,000      17.0 / 19.8   117,000 22.3 / 22.2   160,000 28.0 / 23.6
+// An indoor set's 17 pairs a row (LiDAR: 4.7) move the crossing of 16-bit 64 x 32
+// down; the other limits hold there too (whole layer, here / ring, us):
+//   16-bit 64 x 32    48,000 19.9 / 24.4    90,000 31.9 / 28.7
+//   16-bit 64 x 16   130,000 33.0 / 36.6    32 x 32 260,000 45.1 / 51.4    32 x 64 130,000 27.3 / 30.1
+//   fp32   64 x 16    96,000 47.7 / 56.0    32 x 32 130,000 39.1 / 44.0
 inline bool narrow_ok(int64_t n_src, int64_t n_dst, int K, int Kd, int Nd, size_t esz, bool x3, const void* A) {
   if (Kd > 64 || Nd > 64 || Kd % 4 != 0 || K > kNarrowMaxK) return false;
   if (narrow_chunks(Kd) * narrow_blocks(Nd) * (x3 ? 2 : 1) > 16) return false;  // not built
@@ -78,7 +83,8 @@ inline bool narrow_ok(int64_t n_src, int64_t n_dst, int K, int Kd, int Nd, size_
   if (lds > kNarrowLds) return false;
   if ((Kd == 32 || Kd == 64) && (uintptr_t)A % 16 == 0) {
     const bool fills = 2 * lds > kNarrowLdsCu;
-    return n_dst <= (Kd == 32 ? (fills ? 131072 : 262144) : (fills ? 98304 : 131072));
+    if (Kd == 32) return n_dst <= (fills ? 131072 : 262144);
+    return n_dst <= (fills ? (x3 ? 98304 : 65536) : 131072);
   }
   return true;
 }
