@@ -113,7 +113,7 @@ def _events_batch(torch, fn, reps):
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "hbm_traffic_config2_subm64.md")
 # the sources of the gather and weight-gradient kernels whose counters the traffic file holds
-GEMM_SOURCES = ("gemm_kernels.h", "gemm_wide.h", "gemm_x3.h", "gemm_x3.hip", "mfma.h", "nbr_src.h")
+GEMM_SOURCES = ("gemm_kernels.h", "gemm_wide.h", "gemm_narrow.h", "gemm_x3.h", "gemm_x3.hip", "mfma.h", "nbr_src.h")
 
 
 def gemm_sources_sha():
