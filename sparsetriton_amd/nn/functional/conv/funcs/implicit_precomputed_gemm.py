@@ -81,12 +81,13 @@ def gather_gemm_tiled(A: torch.Tensor, tiles, Bt: torch.Tensor, n_dst: int, K: i
     return out
 
 
+# The narrow gather's LDS for weights.  Larger ones need no library call to learn that the kernel does
+# not take them: at 64 -> 64 and 5,000 rows, where the host sets the pace, the call cost 2 of 27 us.
+_B_KN_BYTES = 112 << 10
+
+
 def b_kn_ok(A: torch.Tensor, n_dst: int, K: int, Nd: int) -> bool:
-    """Whether the tiled gather-GEMM reads W (K, C_in, C_out) itself (no transposed copy).  Weights that
-    cannot fit the kernel's 112 KB of LDS need no library call to say so: at 64 -> 64 and 5,000 rows,
-    where the host sets the pace, the call cost 2 of 27 us."""
-    if K * A.shape[1] * Nd * A.element_size() > 112 << 10:
-        return False
+    """Whether the tiled gather-GEMM reads W (K, C_in, C_out) itself (no transposed copy)."""
     return _lib.lib().st_gather_b_kn_ok(_lib.ptr(A), A.shape[0], n_dst, K, A.shape[1], Nd,
                                         _lib.compute_code(A.dtype)) == 1
 
@@ -104,7 +105,7 @@ def gather_gemm_fwd(A: torch.Tensor, kmap: KernelMap, Bt: torch.Tensor, bias=Non
 def conv_forward(A: torch.Tensor, kmap: KernelMap, W: torch.Tensor, bias=None) -> torch.Tensor:
     """``gather_gemm_fwd`` with the layer's weights W (K, C_in, C_out), transposed first where the
     kernel does not read them as they are."""
-    if b_kn_ok(A, kmap.n_out, kmap.K, W.shape[2]):
+    if W.nbytes <= _B_KN_BYTES and b_kn_ok(A, kmap.n_out, kmap.K, W.shape[2]):
         return gather_gemm_tiled(A, kmap.forward_tiles(), W, kmap.n_out, kmap.K, bias=bias, b_kn=True)
     return gather_gemm_fwd(A, kmap, weight_prep(W, _lib.W_TRANSPOSE), bias=bias)
 
@@ -139,7 +140,7 @@ def conv_forward_epilogue(features: torch.Tensor, weights: torch.Tensor, kmap: K
     dims = (kmap.n_out, K, C_in, C_out, _lib.compute_code(A.dtype))
     stream = _lib.stream_of(A.device)
     if bn is not None:
-        kn = b_kn_ok(A, kmap.n_out, K, C_out)
+        kn = w.nbytes <= _B_KN_BYTES and b_kn_ok(A, kmap.n_out, K, C_out)
         if not kn:
             w = weight_prep(w, _lib.W_TRANSPOSE)
         bw, bb, mean, var = (_f32(t) for t in bn[:4])
