@@ -180,8 +180,12 @@ struct Epi {
     add = b;
     if (col >= Nd) return;
     if (var) {
-      mul = rsqrtf(var[col] + eps) * (scale ? scale[col] : 1.f);
-      add = b * mul + ((shift ? shift[col] : 0.f) - mean[col] * mul);
+      mul = (float)rsqrt((double)(var[col] + eps));  // (rsqrtf is off by a unit for a third of the values)
+      if (scale) mul *= scale[col];
+      float sh = -mean[col] * mul;
+      asm("" : "+v"(sh));  // rounded here, not fused into the sum: the bits of a fold made ahead of the call
+      if (shift) sh += shift[col];
+      add = b * mul + sh;
     } else if (scale) {
       mul = scale[col];
       add = b * mul + (shift ? shift[col] : 0.f);

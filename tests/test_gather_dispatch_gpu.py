@@ -85,3 +85,26 @@ def test_transposed_map_after_an_inference_pass(device, transposed):
         g = torch.sin(torch.arange(y.numel(), device=device, dtype=torch.float32)).view_as(y)
         grads.append(torch.autograd.grad(y, [x, w], g))
     assert torch.equal(grads[0][0], grads[1][0]) and torch.equal(grads[0][1], grads[1][1])
+
+
+@pytest.mark.parametrize("n,cin,cout,dtype", [
+    (1500, 4, 16, torch.bfloat16), (1500, 16, 32, torch.float32), (1500, 32, 20, torch.float16),  # weights in LDS
+    (1500, 64, 64, torch.bfloat16), (1500, 128, 128, torch.float32), (1500, 5, 7, torch.float32),  # ring, pipelined
+    (49153, 128, 128, torch.bfloat16), (49153, 64, 128, torch.float32)])  # wide
+@pytest.mark.parametrize("affine", [True, False])
+def test_batch_norm_in_the_store_has_the_bits_of_folded(device, n, cin, cout, dtype, affine):
+    """The batch norm's own tensors give bit for bit the output of the scale and shift that
+    ``SparseBatchNorm.folded`` makes of them."""
+    from sparsetriton_amd.nn import SparseBatchNorm
+    from sparsetriton_amd.nn.functional import sparse_conv3d_fused
+    sp, W, _, rng = _layer(device, n, cin, cout, dtype, cin + cout)
+    bn = SparseBatchNorm(cout, eps=1e-3, affine=affine).to(device).eval()
+    with torch.no_grad():
+        for t in [bn.running_mean, bn.running_var] + list(bn.parameters()):
+            t.copy_(torch.as_tensor(rng.uniform(0.05, 1.5, cout)))
+        kw = dict(bias=torch.as_tensor(rng.standard_normal(cout), device=device).to(dtype),
+                  residual=torch.as_tensor(rng.standard_normal((n, cout)), device=device).to(dtype), relu=True)
+        got = sparse_conv3d_fused(sp, W, 3, bn=bn.running_affine(), **kw).F
+        scale, shift = bn.folded()
+        want = sparse_conv3d_fused(sp, W, 3, scale=scale, shift=shift, **kw).F
+    assert torch.equal(got, want)
