@@ -543,9 +543,9 @@ int st_gather_gemm(const void* A, int64_t n_src, const int32_t* map, int64_t map
  * the same reference kernels (implicit_precomputed_gemm.py:64-177) --:
  * the workgroup reads its tile's offsets and source rows contiguously
  * instead of gathering map entries and masks row by row.  Same result as
- * st_gather_gemm with that map (up to fp32 rounding for reductions below 32:
- * several offsets then share a matrix instruction).  Reductions wider than 128 (16-bit and
- * ST_F32_BF16X3) or 64 (ST_F32) return ST_ERR_UNSUPPORTED.  flags:
+ * st_gather_gemm with that map (ST_F32_BF16X3 with reductions up to 16: up to
+ * fp32 rounding, several offsets then share a matrix instruction).  Reductions
+ * wider than 128 (16-bit and ST_F32_BF16X3) or 64 (ST_F32) return ST_ERR_UNSUPPORTED.  flags:
  * ST_GATHER_REVERSE_K multiplies offset k's sources by Bt[K - 1 - k] -- the
  * input gradient of a submanifold map that is its own transpose, read over
  * the forward's plan with the weights as given (W (K, C_in, C_out) is then

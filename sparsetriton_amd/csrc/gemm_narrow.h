@@ -23,9 +23,13 @@
 // Kd / 8 chunks per offset rounded up to 1, 2 or 4, lane group g holds chunk
 // g % KC of the step's offset g / KC, so a 16-channel layer runs two offsets
 // per MFMA and a 4-channel layer four (their 16-byte rows are loaded in the
-// MFMA layout as they are).  From 32 elements on a row sums one offset per MFMA
+// MFMA layout as they are).  Of a step's offsets, one that no row of the 16 has
+// takes a slice of zeros in its weights' place: an infinite weight reaches no
+// row group that lacks its offset.  Otherwise a row sums one offset per MFMA
 // in the tile's ascending order (fp32: the three products in the order of
-// mfma_x3), as the ring kernels do, and agrees with them bitwise.
+// mfma_x3).  16-bit sums agree bitwise with the ring and pipelined kernels' at
+// every width, fp32 ones from 17 elements on (below, a step's first products
+// precede its second ones: the same terms, another fp32 order).
 //
 // Bound: at small sizes the chain head -> rows -> products of a wave tile (8 us
 // with the launch up to 20,000 rows), at large ones the gathers' cache lines.
@@ -209,6 +213,7 @@ __global__ __launch_bounds__(64 * NW) void gather_gemm_narrow_kernel(const T* __
   constexpr int D = 4;                            // row loads in flight (steps)
   constexpr int TS = 4;                           // steps per turn
   constexpr int SLICE = KC * NBLK * PLANES * 16;  // 16-byte units of weights per offset
+  constexpr int ZERO = OPS > 1 ? SLICE : 0;       // a slice of zeros after the K of weights
   constexpr int WPT = kGemmBM / 16;               // wave tiles per plan tile
   constexpr int NIX = OPS;                        // index registers per turn (four offsets of 16 rows each)
   constexpr int CH = KC * (X3 ? 2 : 1);           // 16-byte chunks per source row
@@ -222,6 +227,7 @@ __global__ __launch_bounds__(64 * NW) void gather_gemm_narrow_kernel(const T* __
   const int c = lane & 15, g = lane >> 4;
 
   stage_weights<T, KC, NBLK, 64 * NW>(w_s, B, b_kn, K, Kd, Nd);
+  for (int u = tid; u < ZERO; u += 64 * NW) w_s[K * SLICE + u] = F16{};
   __syncthreads();
 
   // every array through 32-bit buffer offsets (the host keeps them below 2 GB)
@@ -237,7 +243,7 @@ __global__ __launch_bounds__(64 * NW) void gather_gemm_narrow_kernel(const T* __
   const F16* const w_lane = w_s + (gq * NBLK * PLANES) * 16 + c;
   // the wave's stage: chunk q of row r of the step's offset o at unit (o * 16 + r) * CH + (q ^ (r / GR % CH)):
   // stores are contiguous, and the 16 rows of a fragment read fall on 16 different 16-byte bank groups
-  v4f* const st = reinterpret_cast<v4f*>(w_s + K * SLICE) + wid * (STAGED ? NI * 64 : 0);
+  v4f* const st = reinterpret_cast<v4f*>(w_s + K * SLICE + ZERO) + wid * (STAGED ? NI * 64 : 0);
   // Loader lanes: load v of a step brings chunk q of row r of the step's offset o, flat = v * 64 + lane =
   // (o * 16 + r) * CH + q (not staged: the MFMA layout, chunk v of row c of offset g).  A chunk past the row's
   // end takes an offset past the buffer's.
@@ -343,10 +349,12 @@ __global__ __launch_bounds__(64 * NW) void gather_gemm_narrow_kernel(const T* __
       constexpr uint64_t lanes = OPS == 4 ? ~0ull : ((1ull << (OPS * 16)) - 1) << L;
       if (!(act[R] & lanes)) return;
       const F16* w = w_lane;
-      if constexpr (OPS == 1)
+      if constexpr (OPS == 1) {
         w += __builtin_amdgcn_readlane(kreg, j);
-      else
-        w += __shfl(kreg, min(j * OPS + go, nk - 1), 64);
+      } else {
+        const int at = __shfl(kreg, min(j * OPS + go, nk - 1), 64);
+        w += (act[R] >> (L + go * 16)) & 0xffff ? at : K * SLICE;
+      }
       F16 bh[KS][NBLK], bl[KS][NBLK];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
@@ -453,7 +461,7 @@ static void launch_narrow_shape(const T* A, int64_t n_src, const TiledSrc& src, 
                                 int b_kn, T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd,
                                 hipStream_t stream) {
   constexpr int STAGE = KC > 1 ? (KC >= 4 ? 1 : 4 / KC) * 16 * KC * (sizeof(T) == 4 ? 2 : 1) * 16 : 0;  // bytes per wave
-  const int w_lds = (int)narrow_lds(K, Kd, Nd, sizeof(T) == 4);
+  const int w_lds = (int)narrow_lds(K + (KC < 4), Kd, Nd, sizeof(T) == 4);  // (up to 16 elements: and the slice of zeros)
   const int64_t wave_tiles = (n_dst + kGemmBM - 1) / kGemmBM * (kGemmBM / 16);
   auto launch = [&](auto nw) {
     constexpr int NW = decltype(nw)::value;

@@ -119,6 +119,51 @@ def test_narrow_gather(device, dtype, n_out, n_in, K, Kd, Nd, density):
     assert np.all(np.abs(y.double().cpu().numpy() - ref) <= bound * 1.001 + 1e-30)
 
 
+SAME_BITS = [(Kd, Nd, dt) for Kd, Nd in [(4, 16), (8, 20), (12, 32), (16, 16), (16, 64), (24, 16), (32, 32), (64, 16)]
+             for dt in (torch.float32, torch.bfloat16, torch.float16) if dt != torch.float32 or Kd > 16]
+
+
+@pytest.mark.parametrize("Kd,Nd,dtype", SAME_BITS)
+@pytest.mark.parametrize("n,density", [(17, 0.9), (1500, 0.15), (3000, 0.6)])
+def test_narrow_gather_sums_like_the_other_kernels(device, dtype, Kd, Nd, n, density):
+    """Bit for bit the sums of the kernels that take rows off its alignment (a view that starts one
+    element into its allocation): offsets in the tile's ascending order.  (fp32 up to 16 elements: the
+    same terms in another fp32 order, bounded by test_narrow_gather.)"""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import b_kn_ok, gather_gemm_tiled
+    rng = np.random.default_rng(Kd + Nd + n)
+    nbr = _map(rng, n, n, 27, density)
+    tiles = _tiled(nbr, n, device)
+    X = torch.as_tensor(rng.standard_normal((n, Kd)), device=device).to(dtype)
+    Wt = torch.as_tensor(rng.standard_normal((27, Nd, Kd)), device=device).to(dtype)
+    view = torch.zeros(n * Kd + 1, dtype=dtype, device=device)[1:].view(n, Kd).copy_(X)
+    assert not b_kn_ok(view, n, 27, Nd)
+    assert torch.equal(gather_gemm_tiled(X, tiles, Wt, n, 27), gather_gemm_tiled(view, tiles, Wt, n, 27))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Kd,Nd", [(4, 16), (8, 32), (16, 20), (16, 32), (32, 32)])
+def test_narrow_gather_contains_non_finite_weights(device, dtype, Kd, Nd):
+    """An infinite weight slice reaches no row of a 16-row group without a source at its offset."""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import gather_gemm_tiled
+    rng = np.random.default_rng(Kd + Nd)
+    n, K, k = 2000, 27, 13
+    nbr = _map(rng, n, n, K, 0.3)
+    nbr[rng.random(n) < 0.97, k] = -1  # few rows use offset k: whole groups lack it, their neighbours have it
+    tiles = _tiled(nbr, n, device)
+    perm = tiles.perm.cpu().numpy()[:n]
+    has = np.add.reduceat(nbr[perm, k] >= 0, np.arange(0, n, 16)) > 0
+    clean = torch.as_tensor(perm[~np.repeat(has, 16)[:n]].astype(np.int64))
+    assert 16 <= len(clean) < n
+    X = torch.as_tensor(rng.standard_normal((n, Kd)), device=device).to(dtype)
+    W = torch.as_tensor(rng.standard_normal((K, Kd, Nd)), device=device).to(dtype)
+    W[k] = 0.0
+    y = gather_gemm_tiled(X, tiles, W, n, K, b_kn=True).cpu()
+    W[k] = float("inf")
+    y2 = gather_gemm_tiled(X, tiles, W, n, K, b_kn=True).cpu()
+    assert torch.equal(y[clean], y2[clean])
+    assert not torch.isfinite(y2[torch.as_tensor(nbr[:, k] >= 0)]).any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("Kd,Nd", [(4, 16), (16, 20), (32, 32)])
 def test_narrow_gather_takes_views_and_contains_non_finite_rows(device, dtype, Kd, Nd):
