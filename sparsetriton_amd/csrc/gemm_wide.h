@@ -95,7 +95,9 @@ __global__ __launch_bounds__(128 * TP) void gather_gemm_wide_kernel(const T* __r
   // B, double-buffered; before the main loop a submanifold source's prologue
   // keeps its unit_rows lookup tables (8 brick words and bases per thread)
   // here too, so the buffer is sized for both
-  constexpr int BT_BYTES = 2 * PLANES * BN * KD * (int)sizeof(L16);
+  // (the pipelined step: and a third buffer, of zeros)
+  constexpr bool PIPE = !X3 && TP == 2;
+  constexpr int BT_BYTES = (PIPE ? 3 : 2) * PLANES * BN * KD * (int)sizeof(L16);
   constexpr int LK_BYTES = S::kTiled ? 0 : 8 * NT * (int)(sizeof(unsigned long long) + sizeof(int32_t));
   __shared__ __attribute__((aligned(16))) unsigned char bt_raw[BT_BYTES > LK_BYTES ? BT_BYTES : LK_BYTES];
   auto bt_s = reinterpret_cast<L16 (*)[PLANES][BN * KD]>(bt_raw);
@@ -304,28 +306,32 @@ __global__ __launch_bounds__(128 * TP) void gather_gemm_wide_kernel(const T* __r
   // B(i + 1) is stored to the other buffer and of B(i + 2) loaded; a k-step's B
   // fragments are read during the one before it.  One barrier a step, one block
   // of straight code: a branch around the products of a wave that lacks the
-  // offset made the compiler move the accumulators between register sets.
+  // offset made the compiler move the accumulators between register sets.  Such
+  // a wave reads its B fragments from a buffer of zeros instead (with the
+  // slice's own, an infinite weight would reach rows that never meet it).
   // 128 x 128, 27 offsets: 150,000 indoor rows 144 -> 123 us, 235,000 LiDAR rows
   // 91 -> 81 us.  (One tile a workgroup keeps the plain step: there other
   // workgroups of the CU fill the gaps, and one step of lead is too short for
   // its loads: 64 -> 128 with lookups 200 -> 207 us.)
-  if constexpr (!X3 && TP == 2) {
+  if constexpr (PIPE) {
     auto pipe_step = [&](int i) {
       constexpr int GROUPS = KSTEPS * MB;
-      const int buf = i & 1, ia = min(i + 1, nk - 1);
+      const int buf = i & 1, ia = min(i + 1, nk - 1), from = any_ring[0] ? buf : 2;
       const int kb = b_slice(src, uk_s[min(i + 2, nk - 1)]);
       int at[MB];
       const int si = pos_s[hw][ia];
+      bool any = false;
 #pragma unroll
       for (int m = 0; m < MB; ++m) {
         const int32_t sv = src_s[hw][max(si, 0)][wt * 64 + m * 16 + c];
+        any |= sv >= 0;
         at[m] = si >= 0 && sv >= 0 ? (sv * KD + g * 8) * (int)sizeof(T) : kOobOffset;
       }
       F16 bh[2][NBLK];
       auto read_b = [&](int s) {
 #pragma unroll
         for (int nb = 0; nb < NBLK; ++nb)
-          bh[s & 1][nb] = *reinterpret_cast<const F16*>(&bt_s[buf][0][bpos(nb * 16 + c, s * 4 + g)]);
+          bh[s & 1][nb] = *reinterpret_cast<const F16*>(&bt_s[from][0][bpos(nb * 16 + c, s * 4 + g)]);
       };
       read_b(0);
       __builtin_amdgcn_sched_barrier(0);  // (without it the compiler rotates the accumulators through register copies)
@@ -347,11 +353,13 @@ __global__ __launch_bounds__(128 * TP) void gather_gemm_wide_kernel(const T* __r
           __builtin_amdgcn_sched_barrier(0);
         }
       }
+      any_ring[0] = __ballot(si >= 0 && any) != 0ull;
       __syncthreads();
     };
     if (nk > 0) {
       issue_b(0);
       issue_a(0, std::integral_constant<int, 0>());
+      for (int j = tid; j < BN * CV; j += NT) *reinterpret_cast<F16*>(&bt_s[2][0][j * 8]) = F16{};
       store_b(0);
       issue_b(min(1, nk - 1));
       __syncthreads();

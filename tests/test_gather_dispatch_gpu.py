@@ -108,3 +108,32 @@ def test_batch_norm_in_the_store_has_the_bits_of_folded(device, n, cin, cout, dt
         scale, shift = bn.folded()
         want = sparse_conv3d_fused(sp, W, 3, scale=scale, shift=shift, **kw).F
     assert torch.equal(got, want)
+
+
+def test_wide_gather_contains_non_finite_weights(device):
+    """An infinite weight slice reaches no row of a 64-row group (a wave's rows) without a source at its
+    offset."""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import gather_gemm_tiled
+    from sparsetriton_amd.nn.functional.conv.kmap import TileMap, TilePlan
+    rng = np.random.default_rng(2)
+    n, K, k = 70001, 27, 13
+    nbr = np.stack([rng.permutation(n) for _ in range(K)], 1).astype(np.int32)
+    nbr[rng.random((n, K)) >= 0.2] = -1
+    nbr[rng.random(n) < 0.9, k] = -1  # few rows use offset k
+    masks = ((nbr >= 0).astype(np.uint64) << np.arange(K, dtype=np.uint64)).sum(1).astype(np.uint32)
+    m = torch.as_tensor(masks.view(np.int32)[:, None].copy(), device=device)
+    nbr_t = torch.as_tensor(np.ascontiguousarray(nbr.T), device=device)
+    perm = TilePlan.build(n, K, m).perm
+    tiles = TileMap.build(nbr_t, n, 1, m, K, perm, n, n)
+    order = perm.cpu().numpy()[:n]
+    has = np.add.reduceat(nbr[order, k] >= 0, np.arange(0, n, 64)) > 0
+    clean = torch.as_tensor(order[~np.repeat(has, 64)[:n]].astype(np.int64))
+    assert 64 <= len(clean) < n // 2
+    X = torch.as_tensor(rng.standard_normal((n, 128)), device=device).bfloat16()
+    Wt = torch.as_tensor(rng.standard_normal((K, 128, 128)), device=device).bfloat16()
+    out = []
+    for v in (0.0, float("inf")):
+        Wt[k] = v
+        out.append(gather_gemm_tiled(X, tiles, Wt, n, K).cpu())
+    assert torch.equal(out[0][clean], out[1][clean])
+    assert not torch.isfinite(out[1][torch.as_tensor(nbr[:, k] >= 0)]).any()
