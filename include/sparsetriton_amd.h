@@ -732,6 +732,14 @@ int st_from_dense(const void* dense, int64_t batches, int64_t sx, int64_t sy, in
 int st_mask_spatial_range(const void* coords, int coord_dtype, int64_t n, const int64_t* limits, uint8_t* mask,
                           st_stream_t stream);
 
+/*
+ * The largest batch index of the rows (coords[:, 0].max() of the reference's
+ * constructor, tensor.py:55-138), in parts: parts[i], i < nparts, is the
+ * largest of a share of them (INT32_MIN for an empty share; int64 indices
+ * saturate).  The host takes their maximum; parts may be pinned host memory.
+ */
+int st_batch_index_max(const void* coords, int coord_dtype, int64_t n, int32_t* parts, int nparts, st_stream_t stream);
+
 /* ------------------------------------------------------------ pooling, upsampling
  *
  * sparse_pooling (nn/functional/spatial.py:26-233): row r of coords goes to

@@ -119,6 +119,7 @@ _SIGNATURES = {
     "st_pool_backward": [_P, _P, _P, _L, _I, _I, _P, _P, _I, _P, _P],
     "st_upsample": [_P, _P, _I, _L, _I, _I, _I, _P, _P, _P],
     "st_upsample_backward": [_P, _L, _I, _I, _I, _P, _P],
+    "st_batch_index_max": [_P, _I, _L, _P, _I, _P],
     "st_bn_workspace": [_L, _I, _I, ctypes.POINTER(_L)],
     "st_bn_forward": [_P, _L, _I, _I, _P, _I, _I, _P, _P, _P, _I, _I, ctypes.c_float, ctypes.c_float, _P, _P, _P,
                       _P, _P, _P, _L, _P, _P],

@@ -95,6 +95,38 @@ __global__ __launch_bounds__(256) void mask_range_kernel(const CT* __restrict__ 
   mask[r] = (x >= x0 && x <= x1 && y >= y0 && y <= y1 && z >= z0 && z <= z1) ? 1 : 0;
 }
 
+// parts[i] = largest batch index of workgroup i's share of the rows (INT32_MIN without one; int64
+// indices saturate).  A few words the host reduces, so nothing has to be set before the launch.
+// Bound: the latency of a thread's loads, so eight of them are in flight (470,532 rows: a loop
+// of one at a time over 64 x 256 threads added 20 us to a 600 us layer).
+template <typename CT>
+__global__ __launch_bounds__(1024) void batch_max_kernel(const CT* __restrict__ coords, int64_t n,
+                                                         int32_t* __restrict__ parts) {
+  __shared__ int32_t wave_s[16];
+  const int64_t step = (int64_t)gridDim.x * 1024;
+  int32_t m = INT32_MIN;
+  for (int64_t r0 = (int64_t)blockIdx.x * 1024 + threadIdx.x; r0 < n; r0 += 8 * step) {
+    CT v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t r = r0 + u * step;
+      v[u] = coords[(r < n ? r : r0) * 4];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int64_t b = v[u];
+      m = max(m, (int32_t)(b > INT32_MAX ? INT32_MAX : (b < INT32_MIN ? INT32_MIN : b)));
+    }
+  }
+  for (int d = 32; d > 0; d >>= 1) m = max(m, __shfl_xor(m, d, 64));
+  if ((threadIdx.x & 63) == 0) wave_s[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) m = max(m, wave_s[w]);
+    parts[blockIdx.x] = m;
+  }
+}
+
 }  // namespace st
 
 using namespace st;
@@ -153,6 +185,13 @@ int st_mask_spatial_range(const void* coords, int coord_dtype, int64_t n, const 
   ST_DISPATCH_COORD(coord_dtype, CT,
                     mask_range_kernel<CT><<<st_blocks(n, 256), 256, 0, stream>>>(
                         (const CT*)coords, n, limits[0], limits[1], limits[2], limits[3], limits[4], limits[5], mask));
+  ST_CHECK_LAUNCH();
+  return ST_OK;
+}
+
+int st_batch_index_max(const void* coords, int coord_dtype, int64_t n, int32_t* parts, int nparts, st_stream_t stream) {
+  if (n < 0 || nparts <= 0 || nparts > 65535 || !parts || (n > 0 && !coords)) return ST_ERR_ARG;
+  ST_DISPATCH_COORD(coord_dtype, CT, batch_max_kernel<CT><<<nparts, 1024, 0, stream>>>((const CT*)coords, n, parts));
   ST_CHECK_LAUNCH();
   return ST_OK;
 }

@@ -23,7 +23,7 @@ import torch
 
 from sparsetriton_amd import _lib
 from sparsetriton_amd.config import ConvAlgo, MIN_TABLE_FACTOR, get_conv_algo, get_h_table_f
-from sparsetriton_amd.tensor import SparseTensor
+from sparsetriton_amd.tensor import SparseTensor, queue_batch_max
 from sparsetriton_amd.utils.hash import HashTable
 
 from .funcs.implicit_hashfly_gemm import (ConvHashOnTheFlyImplicitGEMM, ConvSubmFlyGEMM, InputGradLookup, fly_tile_order,
@@ -159,6 +159,10 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
     # coordinate could not be keyed or the table overflowed -- rows the map would silently lack.
     table_status = None
     in_table = None
+    # New output coordinates are held against the batch size: the brick build has counted the candidates
+    # outside it (max_batch -1); else their largest batch index is read back ahead of the feature kernels.
+    max_batch = None
+    batch_words = None
     if algo == ConvAlgo.PrecomputedNeighborGEMM:
         hit = tensor._cache.neighbor_indices.get(cache_key)
         if hit is not None:
@@ -187,6 +191,7 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
                                                  with_offsets=False)
                 if built is not None:
                     out_coords, new_shape, _, kmap, table_status = built
+                    max_batch = -1
                 else:
                     in_table = _input_table(tensor, scale)
                     out_coords, new_shape, _, kmap, _ = build_out_coords_and_map(
@@ -197,6 +202,8 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
         if out_coords.shape[0] == 0:
             _raise_table_errors(table_status, in_table)
             return _empty(tensor, C_out, new_shape)
+        if not subm_fast and max_batch is None:
+            batch_words, max_batch = queue_batch_max(out_coords), -1
         if hit is None and torch.is_grad_enabled() and (tensor.F.requires_grad or weight.requires_grad):
             # the weight gradient's pair list is built with the tile plan, alongside it
             kmap.forward_tiles(with_pairs=True)
@@ -242,6 +249,8 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
         if out_coords.shape[0] == 0:
             _raise_table_errors(table_status, in_table)
             return _empty(tensor, C_out, new_shape)
+        if not subm_fast:
+            batch_words, max_batch = queue_batch_max(out_coords), -1
         out_feats = ConvHashOnTheFlyImplicitGEMM.apply(
             tensor.F, weight, out_coords, offsets, in_keys, in_vals, lookup_shape,
             1 if transposed else s, tensor.C, gl)
@@ -256,7 +265,9 @@ def _sparse_conv3d(tensor, weight, kernel_size, bias, stride, dilation, padding,
     if submanifold and (out_coords is tensor.C or (out_coords.shape == tensor.C.shape
                                                    and torch.equal(out_coords, tensor.C))):
         return tensor.replace(out_feats)
-    return tensor._derive(out_feats, out_coords, new_shape)
+    if batch_words is not None:
+        max_batch = max(batch_words.values())
+    return tensor._derive(out_feats, out_coords, new_shape, max_batch)
 
 
 def _brick_index(tensor: SparseTensor, eligible: bool, K: int, C_in: int, C_out: int):

@@ -22,7 +22,7 @@ from typing import Tuple
 import torch
 
 from sparsetriton_amd import _lib
-from sparsetriton_amd.tensor import SparseTensor
+from sparsetriton_amd.tensor import BATCH_PARTS, SparseTensor, queue_batch_max
 
 __all__ = ["sparse_pooling", "sparse_upsample"]
 
@@ -44,11 +44,14 @@ class _Pool(torch.autograd.Function):
         seg = torch.empty((n + 1,), dtype=torch.int32, device=dev)
         inv = torch.empty((max(n, 1),), dtype=torch.int32, device=dev)
         oc = torch.empty((max(n, 1), 4), dtype=c.dtype, device=dev)
-        counts = torch.empty((2,), dtype=torch.int32, device=dev)
+        # the plan's counts, then the largest batch index in parts: one read-back for both
+        both = torch.empty((2 + BATCH_PARTS,), dtype=torch.int32, device=dev)
+        both_ptr = _lib.ptr(both)
+        queue_batch_max(c, both_ptr + 8)
         _lib.call("st_pool_plan", _lib.ptr(c), _lib.coord_code(c.dtype), n, int(kernel_size), int(stride),
                   int(padding), _lib.ptr(ws), nbytes.value, _lib.ptr(perm), _lib.ptr(seg), _lib.ptr(inv),
-                  _lib.ptr(oc), _lib.ptr(counts), s)
-        n_out, bad = counts.tolist()
+                  _lib.ptr(oc), both_ptr, s)
+        n_out, bad, *words = both.tolist()
         if bad:
             raise ValueError(f"{bad} pooled cells fall outside the coordinate key range "
                              "(sample index in [0, 32767], spatial values in int16)")
@@ -58,10 +61,10 @@ class _Pool(torch.autograd.Function):
         ctx.save_for_backward(x if mode == "max" else None, out if mode == "max" else None, inv, seg)
         ctx.meta = (n, C, _MODES[mode])
         ctx.mark_non_differentiable(oc)
-        return out, oc[:n_out]
+        return out, oc[:n_out], max(words) if n else -1
 
     @staticmethod
-    def backward(ctx, dout, _dcoords):
+    def backward(ctx, dout, _dcoords, _max_batch):
         x, out, inv, seg = ctx.saved_tensors
         n, C, mode = ctx.meta
         g = dout.contiguous()
@@ -78,8 +81,8 @@ def sparse_pooling(input: SparseTensor, kernel_size: int, padding: int, stride: 
     if stride is None:
         stride = kernel_size
     new_shape = tuple((int(s) - kernel_size + padding * 2) // stride + 1 for s in input.spatial_shape)
-    feats, coords = _Pool.apply(input.F, input.C, kernel_size, padding, stride, mode)
-    return input._derive(feats, coords, new_shape)
+    feats, coords, max_batch = _Pool.apply(input.F, input.C, kernel_size, padding, stride, mode)
+    return input._derive(feats, coords, new_shape, max_batch)
 
 
 class _Upsample(torch.autograd.Function):
@@ -111,6 +114,8 @@ def sparse_upsample(input: SparseTensor, scale_factor: int = None) -> SparseTens
     if scale_factor is None or int(scale_factor) < 1:
         raise ValueError(f"scale_factor must be a positive integer, got {scale_factor}")
     _lib.require_device(input.F, "SparseTensor features")
+    # (each row's batch index goes to all its output rows)
+    words = queue_batch_max(input.C)
     feats, coords = _Upsample.apply(input.F, input.C, int(scale_factor))
     new_shape = tuple(int(s) * int(scale_factor) for s in input.spatial_shape)
-    return input._derive(feats, coords, new_shape)
+    return input._derive(feats, coords, new_shape, -1 if words is None else max(words.values()))

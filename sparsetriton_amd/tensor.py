@@ -17,8 +17,9 @@ from typing import Any, Dict, List, Optional, Tuple, Union
 
 import torch
 
+from sparsetriton_amd import _lib
 from sparsetriton_amd.config import get_coords_dtype
-from sparsetriton_amd.utils.hash import HashTable
+from sparsetriton_amd.utils.hash import HashTable, HostWords
 from sparsetriton_amd.utils.to_dense import to_dense
 
 __all__ = ["SparseTensor", "TensorCache", "randn"]
@@ -33,9 +34,26 @@ class TensorCache:
         self.neighbor_indices: Dict[Tuple[Any, ...], Tuple[torch.Tensor, Any, Tuple]] = {}
 
 
-def _version(t: torch.Tensor) -> Optional[int]:
-    """The tensor's in-place write count; None under inference mode, which keeps none."""
-    return None if t.is_inference() else t._version
+BATCH_PARTS = 64  # workgroups of st_batch_index_max, each leaving one word
+
+
+def queue_batch_max(coords: torch.Tensor, parts_ptr: int = None) -> Optional[HostWords]:
+    """Queues the largest batch index of ``coords`` (as a tensor of them holds it) in BATCH_PARTS int32
+    words, the maximum of which it is: words the host reads without waiting for the work queued
+    since or, with ``parts_ptr``, stored there.  None with nothing to check: no rows, or a stream
+    being captured (a capture reads nothing back; the eager pass before it makes the check)."""
+    if coords.shape[0] == 0 or torch.cuda.is_current_stream_capturing():
+        return None
+    c = coords.to(get_coords_dtype()).contiguous()
+
+    def launch(ptr):
+        _lib.call("st_batch_index_max", _lib.ptr(c), _lib.coord_code(c.dtype), c.shape[0], ptr, BATCH_PARTS,
+                  _lib.stream_of(c.device))
+    return launch(parts_ptr) if parts_ptr else HostWords(BATCH_PARTS, c.device, launch)
+
+
+def _check_batch(batch_size: int, max_b: int) -> None:
+    assert batch_size > max_b, f"batch_size {batch_size} must be > max batch index {max_b}"
 
 
 class SparseTensor:
@@ -70,43 +88,32 @@ class SparseTensor:
             self.batch_size = int(self.coords[:, 0].max().item() + 1) if self.coords.shape[0] > 0 else 0
         else:
             if self.coords.shape[0] > 0:
-                max_b = self.coords[:, 0].max().item()
-                assert batch_size > max_b, f"batch_size {batch_size} must be > max batch index {max_b}"
+                _check_batch(batch_size, self.coords[:, 0].max().item())
             self.batch_size = batch_size
 
         self._cache = TensorCache() if cache is None else cache
-        self._checked_version = _version(self._coords)
 
-    def _coords_checked(self) -> bool:
-        """Whether the coordinates are the ones the constructor checked: not assigned or written since."""
-        return self._checked_version is not None and self._checked_version == _version(self._coords)
-
-    def _derive(self, feats: torch.Tensor, coords: torch.Tensor, spatial_shape) -> "SparseTensor":
-        """A layer's output on new coordinates whose batch indices are this tensor's.  Where those are
-        still the ones the constructor checked (not assigned or written since), nothing is read back
-        from the device: the constructor's check waits for the stream, which in a training step
-        leaves the GPU idle between the forward and the backward."""
-        if not self._coords_checked():
+    def _derive(self, feats: torch.Tensor, coords: torch.Tensor, spatial_shape,
+                max_batch: Optional[int] = None) -> "SparseTensor":
+        """A layer's output on new coordinates, in this tensor's batch.  ``max_batch`` is the largest batch
+        index among them where the layer has it from this very pass (-1: all refused that are not
+        below the batch size, or nothing to check).  Without it the constructor looks for itself and
+        waits for the whole stream, which in a training step leaves the GPU idle between the forward
+        and the backward; a layer reads the index ahead of its feature kernels instead.  (Nothing
+        about the input tensor stands for the check: its batch size is an attribute, and a write to
+        its coordinates need not show in torch's write count.)"""
+        if max_batch is None or self.batch_size is None:
             return SparseTensor(feats, coords, spatial_shape=spatial_shape, batch_size=self.batch_size)
+        _check_batch(self.batch_size, max_batch)
         out = SparseTensor.__new__(SparseTensor)
         out.feats = feats
         out.coords = coords.to(device=feats.device, dtype=get_coords_dtype())
         out.spatial_shape = torch.Size([int(s) for s in spatial_shape])
         out.batch_size = self.batch_size
         out._cache = TensorCache()
-        out._checked_version = _version(out._coords)
         return out
 
     # ------------------------------------------------------------ accessors
-    @property
-    def coords(self) -> torch.Tensor:
-        return self._coords
-
-    @coords.setter
-    def coords(self, coords: torch.Tensor) -> None:
-        self._coords = coords
-        self._checked_version = None  # (see _derive)
-
     @property
     def F(self) -> torch.Tensor:
         return self.feats
@@ -125,11 +132,8 @@ class SparseTensor:
 
     # ------------------------------------------------------------ conversions
     def to(self, device: Union[str, torch.device], non_blocking: bool = False) -> "SparseTensor":
-        checked = self._coords_checked()
         self.feats = self.feats.to(device, non_blocking=non_blocking)
         self.coords = self.coords.to(device, non_blocking=non_blocking)
-        if checked:
-            self._checked_version = _version(self._coords)
         return self
 
     def cpu(self) -> "SparseTensor":
@@ -160,8 +164,6 @@ class SparseTensor:
         out.spatial_shape = self.spatial_shape
         out.batch_size = self.batch_size
         out._cache = self._cache
-        if self._coords_checked():
-            out._checked_version = _version(out._coords)
         return out
 
     def __repr__(self) -> str:

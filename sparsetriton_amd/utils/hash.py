@@ -71,6 +71,31 @@ class StatusSnapshot:
             )
 
 
+class HostWords:
+    """int32 words that one kernel, queued by ``launch(pointer)``, stores straight into pinned host
+    memory: no copy in the stream (a StatusSnapshot's takes 10 us of it).  ``values()`` waits for
+    that kernel only; the memory is held until it has run."""
+
+    _event = None
+
+    def __init__(self, n: int, device: torch.device, launch):
+        self._host = torch.empty((n,), dtype=torch.int32, pin_memory=True)
+        launch(self._host.data_ptr())
+        self._event = torch.cuda.Event()
+        self._event.record(torch.cuda.current_stream(device))
+
+    def values(self) -> list:
+        self._wait()
+        return self._host.tolist()
+
+    def _wait(self) -> None:
+        if self._event is not None:
+            self._event.synchronize()
+            self._event = None
+
+    __del__ = _wait
+
+
 def flatten_coord(coords: torch.Tensor) -> torch.Tensor:
     """Pack (N, 4) rows (b, x, y, z) into int64 ``b<<48 | x<<32 | y<<16 | z`` (``hash.py:25-54``)."""
     c = coords.to(torch.int64)

@@ -134,3 +134,12 @@ def test_derived_tensors_check_coordinates_written_since():
         t.C[1, 0] = 5
         with pytest.raises(AssertionError, match="max batch index"):
             t._derive(f, t.C, (4, 4, 4))
+
+
+def test_saved_tensors_keep_their_fields():
+    """A tensor's state is its plain attributes (what files saved from it hold)."""
+    import pickle
+    t = SparseTensor(torch.zeros(3, 4), C3, spatial_shape=(10, 10, 10), batch_size=2)
+    assert set(vars(t)) == {"feats", "coords", "spatial_shape", "batch_size", "_cache"}
+    u = pickle.loads(pickle.dumps(t))
+    assert torch.equal(u.C, t.C) and u.batch_size == 2 and u.replace(u.F).batch_size == 2
