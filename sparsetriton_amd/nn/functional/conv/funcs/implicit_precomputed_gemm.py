@@ -114,15 +114,34 @@ def _f32(t):
     return None if t is None else t.detach().to(torch.float32).contiguous()
 
 
+_CHANNEL_TERMS = ("bias", "scale", "shift", "bn weight", "bn bias", "running_mean", "running_var")
+
+
+def _check_channel_terms(C_out: int, device: torch.device, bias, scale, shift, bn) -> None:
+    """The kernel reads C_out values behind each of these pointers."""
+    terms = (bias, scale, shift)
+    if bn is not None:
+        if scale is not None or shift is not None:
+            raise ValueError("give either bn or scale / shift")
+        if bn[2] is None or bn[3] is None:
+            raise ValueError("bn needs running_mean and running_var")
+        terms += tuple(bn[:4])
+    for i, t in enumerate(terms):
+        if t is not None and (t.numel() != C_out or t.device != device):
+            raise ValueError(f"{_CHANNEL_TERMS[i]} must hold {C_out} values on {device}, got {tuple(t.shape)} on "
+                             f"{t.device}")
+
+
 def conv_forward_epilogue(features: torch.Tensor, weights: torch.Tensor, kmap: KernelMap, bias, scale, shift,
                           residual, relu: bool, bn=None) -> torch.Tensor:
     """Forward with the store epilogue ``act((sum + bias) * scale + shift + residual)`` (inference:
     no autograd).  ``scale`` / ``shift`` fp32 (C_out) or None; ``bn`` = (weight, bias, running_mean,
     running_var, eps) instead folds an evaluation-mode batch norm inside the kernel; ``bias`` and
     ``residual`` (N_out, C_out) in the features' dtype, residual rows in output order."""
-    _lib.require_device(features, "features")
     N_in, C_in = features.shape
     K, C_in_w, C_out = weights.shape
+    _check_channel_terms(C_out, features.device, bias, scale, shift, bn)
+    _lib.require_device(features, "features")
     assert C_in_w == C_in, f"weights C_in ({C_in_w}) != features C_in ({C_in})"
     assert kmap.K == K, f"kernel map has {kmap.K} offsets, weights {K}"
     if not tiled_ok(features.dtype, C_in):
