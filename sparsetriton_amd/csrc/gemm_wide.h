@@ -59,7 +59,7 @@ struct FlySrc {
 };
 
 // ST_GATHER_WIDE=0 keeps the four-wave kernels everywhere, =2 takes the wide one
-// for every width it is built for (A/B timing); default: 128 x 128 only.
+// for every width it is built for (A/B timing); default: where wide_ok says it is faster.
 inline int gather_wide_mode() {
   static int mode = -1;
   if (mode < 0) {
@@ -408,16 +408,29 @@ __global__ __launch_bounds__(128 * TP) void gather_gemm_wide_kernel(const T* __r
 // (32-bit buffer offsets).  And enough rows: a wide workgroup covers one or two
 // row tiles and all columns, so a deep stage's few thousand rows leave most CUs
 // idle, where the ring kernels launch two to four times the workgroups (same
-// sums, bit for bit).  Ring / wide, us, indoor voxels (17 pairs a row; a LiDAR
-// set's 4.7 move the crossing up, to over 60,000 rows):
-//   16-bit 128 x 128   9,400 rows 35 / 62   28,700 43 / 64   60,000  75 / 66
-//   fp32    64 x 128   9,400      49 / 85   28,700 61 / 90   60,000 101 / 96
-//   fp32   128 x  64   9,400      88 / 110  28,700 94 / 113  60,000 153 / 127
+// sums, bit for bit).  The crossing moves with the pairs a row has, which the
+// host does not know; ring / wide, us, at indoor (17 pairs a row) and LiDAR
+// (4.7) voxels:
+//   rows                 32,000   40,960   49,000   60,000   72,000   90,000   117,000  150,000
+//   16-bit 128 x 128
+//     indoor             47/52    65/52    73/55    76/55    93/85    106/88            166/131
+//     LiDAR              38/48    39/49    39/48    39/47    43/49    49/49    58/52    76/66
+//   fp32 128 x 64
+//     indoor             90/110   136/117  147/118  151/120  199/170  212/179
+//     LiDAR              89/106   89/112   89/111   87/109   89/112   103/115  120/113  156/121
+//   fp32 64 x 128
+//     indoor             59/87    86/92    93/91    98/91    120/130  135/139  172/150  214/199
+//     LiDAR              52/86    52/87    52/87    52/86    54/87    62/88    74/88    95/90
+// At 16 bits and at fp32 128 x 64 the limit lies between the two crossings
+// (either way one of the sets loses up to a third), nearer the dense one: layers
+// of 128 channels sit behind strided stages, where rows have 13 to 17 pairs.  At
+// fp32 64 x 128 the dense sets cross a second time near 95,000 rows and gain at
+// most 10 % before, while sparse ones lose 30 to 65 %: the limit is there.
 inline bool wide_ok(int Kd, int Nd, int K, size_t esz, bool x3, int64_t n_src, int64_t n_dst, const void* A,
                     const void* Bt) {
   const bool built = (Kd == 64 || Kd == 128) && (Nd == 64 || Nd == 128);
   const bool faster = (x3 ? ((Kd == 128) != (Nd == 128)) : (Kd == 128 && Nd == 128)) &&
-                      n_dst > (x3 && Kd == 128 ? 40960 : 49152);
+                      n_dst > (x3 ? (Kd == 128 ? 40960 : 98304) : 49152);
   return built && (faster || gather_wide_mode() == 2) && K <= kWideMaxK && (uintptr_t)A % 16 == 0 &&
          (uintptr_t)Bt % 16 == 0 && n_src * Kd * (int64_t)esz < (1ll << 31) - 64 &&
          (int64_t)K * Nd * Kd * (int64_t)esz < (1ll << 31) - 64;

@@ -714,8 +714,8 @@ def test_fused_epilogue_without_sources(device):
 def test_reverse_k_gather_equals_reversed_weights(device, dtype, C):
     """The input gradient of a symmetric submanifold map over the forward's plan with the weights'
     offsets reversed as the GEMM addresses them (ST_GATHER_REVERSE_K) equals the same gather over
-    an ST_W_REVERSE copy of the weights, bit for bit (ring kernels at 32 / 64 channels, the wide
-    kernel at 128 x 128 16-bit and 64 x 128 split fp32)."""
+    an ST_W_REVERSE copy of the weights, bit for bit (weights in LDS at 32 channels, ring kernels at 64
+    and 128; the wide kernels, which start at more rows: test_gather_dispatch_gpu)."""
     from sparsetriton_amd import _lib
     from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import gather_gemm_tiled, weight_prep
     from sparsetriton_amd.nn.functional.conv.kmap import _target_offsets, subm_kernel_map

@@ -90,7 +90,7 @@ def test_transposed_map_after_an_inference_pass(device, transposed):
 @pytest.mark.parametrize("n,cin,cout,dtype", [
     (1500, 4, 16, torch.bfloat16), (1500, 16, 32, torch.float32), (1500, 32, 20, torch.float16),  # weights in LDS
     (1500, 64, 64, torch.bfloat16), (1500, 128, 128, torch.float32), (1500, 5, 7, torch.float32),  # ring, pipelined
-    (49153, 128, 128, torch.bfloat16), (49153, 64, 128, torch.float32)])  # wide
+    (49153, 128, 128, torch.bfloat16), (98305, 64, 128, torch.float32)])  # wide
 @pytest.mark.parametrize("affine", [True, False])
 def test_batch_norm_in_the_store_has_the_bits_of_folded(device, n, cin, cout, dtype, affine):
     """The batch norm's own tensors give bit for bit the output of the scale and shift that
@@ -137,3 +137,39 @@ def test_wide_gather_contains_non_finite_weights(device):
         out.append(gather_gemm_tiled(X, tiles, Wt, n, K).cpu())
     assert torch.equal(out[0][clean], out[1][clean])
     assert not torch.isfinite(out[1][torch.as_tensor(nbr[:, k] >= 0)]).any()
+
+
+@pytest.mark.parametrize("cin,cout,dtype,last_ring", [
+    (128, 128, torch.bfloat16, 49152), (128, 128, torch.float16, 49152), (64, 128, torch.float32, 98304),
+    (128, 64, torch.float32, 40960)])
+@pytest.mark.parametrize("beyond", [0, 1])
+def test_wide_and_ring_gathers_meet_with_an_epilogue_and_reversed_offsets(device, cin, cout, dtype, last_ring, beyond):
+    """The last row count of the ring kernels and the first of the wide ones: batch norm, residual and ReLU
+    in the store against float64 at the first and last rows (the plain sum's bound through the affine
+    map, and four fp32 roundings of its terms), and reversed offsets, bit for bit those of a reversed
+    copy of the weights."""
+    from sparsetriton_amd import _lib
+    from sparsetriton_amd.nn.functional import sparse_conv3d_fused
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import gather_gemm_tiled, weight_prep
+    n = last_ring + beyond
+    sp, W, nbr, rng = _layer(device, n, cin, cout, dtype, 4)
+    w, b, mean, var = (torch.as_tensor(rng.uniform(lo, 1.5, cout).astype(np.float32), device=device)
+                       for lo in (-1.5, -1.5, -1.5, 0.1))
+    R = torch.as_tensor(rng.standard_normal((n, cout)), device=device).to(dtype)
+    with torch.no_grad():
+        y = sparse_conv3d_fused(sp, W, 3, residual=R, relu=True, bn=(w, b, mean, var, 1e-5)).F
+    w, b, mean, var = (t.double().cpu().numpy() for t in (w, b, mean, var))
+    mul = w / np.sqrt(var + 1e-5)
+    rows = np.r_[0:500, n - 500:n]
+    Xd, Wd, res = sp.F.double().cpu().numpy(), W.double().cpu().numpy(), R[rows].double().cpu().numpy()
+    s, mag = O.fwd_f64_blas(Xd, Wd, nbr[rows]), O.fwd_f64_blas(np.abs(Xd), np.abs(Wd), nbr[rows])
+    ref = np.maximum(s * mul + (b - mean * mul) + res, 0)
+    u = {torch.float32: 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    bound = (27 * cin * 2.0 ** -24 + (2.0 ** -15 if dtype == torch.float32 else 0)) * mag * np.abs(mul) + u * np.abs(ref)
+    bound += 4 * 2.0 ** -24 * (np.abs(s * mul) + np.abs(b) + np.abs(mean * mul) + np.abs(res))
+    assert np.all(np.abs(y[rows].double().cpu().numpy() - ref) <= 1.001 * bound)
+    (_, km, _), = sp._cache.neighbor_indices.values()
+    assert km.symmetric
+    Bt = weight_prep(W, _lib.W_TRANSPOSE)
+    rev = gather_gemm_tiled(sp.F, km.forward_tiles(), Bt, n, 27, reverse_k=True)
+    assert torch.equal(rev, gather_gemm_tiled(sp.F, km.forward_tiles(), Bt.flip(0).contiguous(), n, 27))
