@@ -202,3 +202,60 @@ def test_narrow_gather_refuses_other_shapes(device, dtype, kw):
     assert _lib.lib().st_gather_b_kn_ok(*args) == 0
     assert _lib.lib().st_gather_b_kn_ok(None, 100, 100, 27, 16, 16, _lib.compute_code(dtype)) == 1
     assert _lib.lib().st_gather_b_kn_ok(None, 1 << 27, 100, 27, 16, 16, _lib.compute_code(dtype)) == 0
+
+
+# n_out, Kd, Nd, dtype: sizes at which a workgroup's waves are sixteen (weights over half a CU's LDS, above
+# 32,768 rows) or take a second and third 16-row tile (above 16 rows for each of the resident waves)
+SEVERAL = [
+    (40003, 32, 32, torch.float32), (40003, 64, 32, torch.bfloat16), (65536, 64, 32, torch.float16),  # sixteen waves
+    (70003, 32, 32, torch.float32), (131057, 32, 32, torch.float32), (70003, 16, 64, torch.float32),  # and two tiles
+    (70003, 32, 32, torch.bfloat16), (100003, 16, 16, torch.float32), (140003, 4, 16, torch.bfloat16),  # two tiles
+    (300001, 4, 16, torch.float32), (300001, 16, 16, torch.bfloat16), (131071, 64, 16, torch.float16)]  # three, two
+
+
+def _mixed_map(rng, n, K):
+    """Rows with no, few, some and all sources, in an order that mixes them."""
+    nbr = np.stack([rng.permutation(n) for _ in range(K)], 1).astype(np.int32)
+    nbr[rng.random((n, K)) >= rng.choice([0.0, 0.04, 0.3, 1.0], n, p=[0.1, 0.5, 0.3, 0.1])[:, None]] = -1
+    return nbr
+
+
+@pytest.mark.parametrize("n,Kd,Nd,dtype", SEVERAL)
+@pytest.mark.parametrize("epilogue", [False, True])
+def test_narrow_gather_several_tiles_a_wave(device, n, Kd, Nd, dtype, epilogue):
+    """The loop over a wave's tiles (the next one's head loaded a tile ahead, its count two ahead) and the
+    sixteen-wave form, plain and with a batch norm, a residual and ReLU in the store; rows from both
+    ends and the middle of the tile order and at random against float64 (bound: test_narrow_gather's,
+    through the affine map; its own roundings are four of the terms')."""
+    from sparsetriton_amd.nn.functional.conv.funcs.implicit_precomputed_gemm import b_kn_ok, conv_forward, conv_forward_epilogue
+    rng = np.random.default_rng(n + Kd + Nd)
+    K = 27
+    nbr = _mixed_map(rng, n, K)
+    kmap = _kmap(nbr, n, device)
+    X = torch.as_tensor(rng.standard_normal((n, Kd)), device=device).to(dtype)
+    W = torch.as_tensor(rng.standard_normal((K, Kd, Nd)), device=device).to(dtype)
+    assert b_kn_ok(X, n, K, Nd)
+    mul, add, add_mag = np.ones(Nd), np.zeros(Nd), np.zeros(Nd)
+    if epilogue:
+        w, b, mean = (torch.as_tensor(rng.uniform(-1, 1, Nd).astype(np.float32), device=device) for _ in range(3))
+        var = torch.as_tensor(rng.uniform(0.1, 2, Nd).astype(np.float32), device=device)
+        R = torch.as_tensor(rng.standard_normal((n, Nd)), device=device).to(dtype)
+        y = conv_forward_epilogue(X, W, kmap, None, None, None, R, True, bn=(w, b, mean, var, 1e-5))
+        mul = (w.double() / torch.sqrt(var.double() + 1e-5)).cpu().numpy()
+        b, mean = b.double().cpu().numpy(), mean.double().cpu().numpy()
+        add, add_mag = b - mean * mul, np.abs(b) + np.abs(mean * mul)
+    else:
+        y = conv_forward(X, kmap, W)
+    order = kmap.forward_tiles().perm.cpu().numpy()[:n]
+    rows = np.r_[order[:300], order[n // 2 - 150:n // 2 + 150], order[-300:], rng.integers(0, n, 300)]
+    Xd, Wd = X.double().cpu().numpy(), W.double().cpu().numpy()
+    s, mag = O.fwd_f64_blas(Xd, Wd, nbr[rows]), O.fwd_f64_blas(np.abs(Xd), np.abs(Wd), nbr[rows])
+    bound = ((K * Kd + 2) * 2.0 ** -24 + (2.0 ** -15 if dtype == torch.float32 else 0)) * mag
+    ref = s * mul + add
+    bound = bound * np.abs(mul) + (4 * 2.0 ** -24 * (np.abs(s * mul) + add_mag) if epilogue else 0)
+    if epilogue:
+        res = R[torch.as_tensor(rows)].double().cpu().numpy()
+        ref = np.maximum(ref + res, 0)
+        bound += 2.0 ** -24 * np.abs(res)
+    got = y[torch.as_tensor(rows)].double().cpu().numpy()
+    assert np.all(np.abs(got - ref) <= 1.001 * bound + EPS[dtype] * np.abs(ref) + 1e-30)
