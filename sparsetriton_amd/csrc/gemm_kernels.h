@@ -939,8 +939,13 @@ __global__ __launch_bounds__(256) void wgrad_pairs_f32_kernel(const float* __res
 // through LDS once per chunk.  Needs C_in and C_out multiples of 4, 16-byte
 // aligned arrays below 2 GB; anything else takes the kernel above, which loads
 // every operand element on its own behind its pair's index load: it spent its
-// time waiting on those serial loads (1.2 M pairs at 32 x 32 channels:
-// 119 us there, 43 us here; 2.2 M pairs at 4 x 16: 162 us there, 27 us here).
+// time waiting on those serial loads.  There / here, us, with the reduction:
+//   1.2 M pairs at 32 x 32 119 / 43;  2.2 M (470,532 LiDAR rows) at 4 x 16 162 / 27,
+//   16 x 64 229 / 86, 20 x 36 402 / 120, 48 x 48 756 / 224, 128 x 20 604 / 233,
+//   and in IEEE mode 64 x 64 516 / 280, 128 x 128 1805 / 992
+//   4,096 rows: 64 x 20 39 / 23, 48 x 80 118 / 23, IEEE 64 x 64 51 / 33
+// The LDS holds eight workgroups on a CU at 16 x 16 and three at 32 x 32, and one
+// at 64 x 64 (the launch bound there caps registers only).
 constexpr int stage_pitch_f32(int width) { return width == 16 ? 16 : width + 16; }
 template <int MB, int NB>
 __global__ __launch_bounds__(256, MB + NB > 4 ? 2 : 3) void wgrad_pairs_f32_rows_kernel(
@@ -1773,8 +1778,6 @@ static int launch_gather_e(const T* A, int64_t n_src, const Src& src, const uint
   return ST_OK;
 }
 
-// The general store epilogue (affine map, residual, ReLU) runs on the tiled
-// kernels only; everything else stores acc + bias.
 // Kernels that hold the whole weight tensor in LDS take the narrow layers of a
 // tile plan (gemm_narrow.h); b_kn: B is W (K, Kd, Nd) as the layer stores it,
 // not (K, Nd, Kd).
@@ -1786,6 +1789,8 @@ static int gather_narrow(const T* A, int64_t n_src, const TiledSrc& src, const i
   return ST_OK;
 }
 
+// The general store epilogue (affine map, residual, ReLU) runs on the tiled
+// kernels only; everything else stores acc + bias.
 template <typename T, typename Src>
 static int launch_gather(const T* A, int64_t n_src, const Src& src, const uint32_t* masks, int W,
                          const int32_t* rows, const T* Bt, T* out, Epi<T> epi, int64_t n_dst, int K, int Kd, int Nd,
@@ -2090,8 +2095,8 @@ static void launch_wgrad_pairs_f32(const float* X, const float* dY, const int2* 
       X, dY, pairs, kstart, cstart, chunk_order, K, chunk, Cin, Cout, partials);
 }
 
-// (one workgroup per chunk up to two rounds of chunks at four workgroups per CU: a chunk is short, and
-// the hardware fills the CUs as workgroups end)
+// (one workgroup per chunk up to 2048, which fill the chip at every tile: a chunk is short, and the
+// hardware fills the CUs as workgroups end)
 template <int MB, int NB>
 static void launch_wgrad_pairs_f32_rows(const float* X, int64_t n_in, const float* dY, int64_t n_out, const int2* pairs,
                                         const int32_t* kstart, const int32_t* cstart, const int32_t* chunk_order, int K,

@@ -62,7 +62,15 @@ inline int64_t narrow_lds(int K, int Kd, int Nd, bool x3) {
 // groups aligned to them, the arrays lie within 32-bit buffer offsets and the
 // weights within the LDS.  Reductions the ring kernels are not built for (Kd
 // other than 32 and 64) always come here: the alternative is the one-offset
-// pipelined kernel.  At 32 and 64 the ring kernels win once the rows keep their
+// pipelined kernel, which was nowhere faster (here / there, us):
+//                     470,532 LiDAR rows        300,000 / 900,000 indoor rows
+//   fp32   16 x 64     69 / 136                  69 / 188,  258 / 491
+//          20 x 32     58 / 98                   67 / 131,  272 / 353
+//          40 x 16     80 / 123                 109 / 184,  390 / 495
+//   16-bit  8 x 64     32 / 78                   33 / 103,  112 / 252
+//          24 x 32     37 / 68                   44 / 78,   180 / 219
+//          48 x 32     55 / 92                   66 / 130,  273 / 333
+// At 32 and 64 the ring kernels win once the rows keep their
 // larger tiles busy, so there the kernel takes sets up to a size, smaller where
 // the weights fill a CU's LDS (one workgroup on a CU) and for the longer rows
 // (here / ring, us, LiDAR voxels):
