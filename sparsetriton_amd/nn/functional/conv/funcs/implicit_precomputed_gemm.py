@@ -111,7 +111,9 @@ def conv_forward(A: torch.Tensor, kmap: KernelMap, W: torch.Tensor, bias=None) -
 
 
 def _f32(t):
-    return None if t is None else t.detach().to(torch.float32).contiguous()
+    if t is None or (t.dtype == torch.float32 and t.is_contiguous()):
+        return t
+    return t.detach().to(torch.float32).contiguous()
 
 
 _CHANNEL_TERMS = ("bias", "scale", "shift", "bn weight", "bn bias", "running_mean", "running_var")
@@ -253,8 +255,8 @@ def window_wgrad_ok(X: torch.Tensor, dY: torch.Tensor, kmap: KernelMap) -> bool:
     """Whether the weight gradient runs over the map itself (st_wgrad's window kernel, the map's
     columns in ``window_order``) instead of the pair list: only when ST_WGRAD_PATH=window asks
     for it, for 16-bit rows with C_in and C_out multiples of 128.  On config 5 (1 M rows, 18
-    pairs a row) it moves half the fabric bytes of the pair-list kernel (2.6 vs 5.2 GB) at the
-    same time (1.05 vs 1.04 ms), so the pair list stays the default."""
+    pairs a row) it moves fewer fabric bytes than the pair-list kernel (2.6 vs 4.4 GB) but takes
+    longer (1.05 vs 0.78 ms), so the pair list stays the default."""
     if os.environ.get("ST_WGRAD_PATH", "pairs") != "window":
         return False
     return X.dtype in (torch.bfloat16, torch.float16) and X.shape[1] % 128 == 0 and dY.shape[1] % 128 == 0
