@@ -153,6 +153,14 @@ __device__ __forceinline__ T from_f32(float v) {
   return (T)v;
 }
 
+// 1 / sqrt(x) rounded to nearest (but for one value in ten million; rsqrtf is a unit off for a third
+// of them): one Newton step whose residual 1 - x r^2 keeps the rounding of x r.
+__device__ __forceinline__ float rsqrt_rn(float x) {
+  const float r = rsqrtf(x), h = x * r, l = fmaf(x, r, -h);
+  const float e = fmaf(-l, r, fmaf(-h, r, 1.f));
+  return e == e ? fmaf(0.5f * r, e, r) : r;  // (r infinite or zero: no step)
+}
+
 // Store epilogue of the gather-GEMMs, on the fp32 accumulator of (row r, column c):
 //   v = (acc + bias[c]) * mul[c] + add[c] + residual[r, c], then ReLU when relu is set
 // bias (the convolution's, conv.py:227-228) and residual (n_dst x Nd, rows in
@@ -180,12 +188,12 @@ struct Epi {
     add = b;
     if (col >= Nd) return;
     if (var) {
-      mul = (float)rsqrt((double)(var[col] + eps));  // (rsqrtf is off by a unit for a third of the values)
-      if (scale) mul *= scale[col];
-      float sh = -mean[col] * mul;
+      // (all loads first: a column's chain of them is what this costs)
+      const float vr = var[col], m = mean[col], w = scale ? scale[col] : 1.f, t = shift ? shift[col] : 0.f;
+      mul = rsqrt_rn(vr + eps) * w;
+      float sh = -m * mul;
       asm("" : "+v"(sh));  // rounded here, not fused into the sum: the bits of a fold made ahead of the call
-      if (shift) sh += shift[col];
-      add = b * mul + sh;
+      add = b * mul + (sh + t);
     } else if (scale) {
       mul = scale[col];
       add = b * mul + (shift ? shift[col] : 0.f);

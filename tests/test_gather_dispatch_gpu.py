@@ -173,3 +173,22 @@ def test_wide_and_ring_gathers_meet_with_an_epilogue_and_reversed_offsets(device
     Bt = weight_prep(W, _lib.W_TRANSPOSE)
     rev = gather_gemm_tiled(sp.F, km.forward_tiles(), Bt, n, 27, reverse_k=True)
     assert torch.equal(rev, gather_gemm_tiled(sp.F, km.forward_tiles(), Bt.flip(0).contiguous(), n, 27))
+
+
+def test_batch_norm_in_the_store_at_extreme_variances(device):
+    """Variances from subnormal to huge, zero and infinite (eps 0): the bits of ``folded``."""
+    from sparsetriton_amd.nn import SparseBatchNorm
+    from sparsetriton_amd.nn.functional import sparse_conv3d_fused
+    n, C = 300, 64
+    sp, W, _, rng = _layer(device, n, 16, C, torch.float32, 11)
+    bn = SparseBatchNorm(C, eps=0.0, affine=False).to(device).eval()
+    for round_ in range(40):
+        var = (10.0 ** rng.uniform(-37, 38, C)).astype(np.float32)
+        if round_ == 0:
+            var[:4] = (0.0, np.inf, 1e-40, np.float32(2.0) ** -126)
+        bn.running_var.copy_(torch.as_tensor(var))
+        with torch.no_grad():
+            got = sparse_conv3d_fused(sp, W, 3, bn=bn.running_affine()).F
+            scale, shift = bn.folded()
+            want = sparse_conv3d_fused(sp, W, 3, scale=scale, shift=shift).F
+        assert torch.equal(torch.nan_to_num(got), torch.nan_to_num(want)) and torch.equal(got.isnan(), want.isnan())
