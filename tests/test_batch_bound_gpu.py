@@ -84,3 +84,30 @@ def test_batch_index_max(device, dtype, n):
     host = HostWords(64, c.device, lambda ptr: _lib.call("st_batch_index_max", _lib.ptr(c), _lib.coord_code(dtype), n,
                                                          ptr, 64, _lib.stream_of(c.device)))
     assert max(host.values()) == want == max(host.values())
+
+
+def test_layers_over_cached_maps_can_be_captured(device):
+    """A graph takes a strided convolution over a cached map and an upsampling (the eager pass before it
+    checked their batch indices); every replay equals the eager result."""
+    t = _tensor(device)
+    w = torch.ones((27, 16, 8), device=device)
+    x = torch.randn_like(t.F)
+
+    def run():
+        with torch.no_grad():
+            y = sparse_conv3d(t.replace(x), w, 3, stride=2, padding=1, submanifold=False)
+            return sparse_upsample(y, 2).F
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        run()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = run()
+    for seed in range(3):
+        x.copy_(torch.randn(x.shape, generator=torch.Generator().manual_seed(seed)))
+        want = run()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
