@@ -113,6 +113,13 @@ class SparseTensor:
         out._cache = TensorCache()
         return out
 
+    def __setstate__(self, state: dict) -> None:
+        # (saved while the coordinates were kept under another name)
+        if "_coords" in state:
+            state = {k: v for k, v in state.items() if k != "_checked_version"}
+            state["coords"] = state.pop("_coords")
+        self.__dict__.update(state)
+
     # ------------------------------------------------------------ accessors
     @property
     def F(self) -> torch.Tensor:

@@ -143,3 +143,7 @@ def test_saved_tensors_keep_their_fields():
     assert set(vars(t)) == {"feats", "coords", "spatial_shape", "batch_size", "_cache"}
     u = pickle.loads(pickle.dumps(t))
     assert torch.equal(u.C, t.C) and u.batch_size == 2 and u.replace(u.F).batch_size == 2
+    v = SparseTensor.__new__(SparseTensor)
+    v.__setstate__({"feats": t.F, "_coords": t.C, "spatial_shape": t.spatial_shape, "batch_size": 2, "_cache": t._cache,
+                    "_checked_version": 0})
+    assert set(vars(v)) == set(vars(t)) and torch.equal(v.C, t.C)
